@@ -112,8 +112,9 @@ struct gta_ctx {
     // pair state
     DevBuf s_flags, s_grand, s_best0, s_prev, s_naln, s_qpos, s_rpos, s_fndx, s_fpos;
     DevBuf s_tibest, s_tgrand, s_out, s_aln, s_btck, s_btckoff, s_rowbuf, s_cells, s_alns, s_algb;
-    // DP size buckets: pairs filled by W waves (and their ring rows)
-    DevBuf s_dpsmall, s_dpbig, s_ring, s_ringoff, s_fail, s_gstrip0, s_gsync;
+    // DP forms: pair lists, and the rows, row offsets, first strips and item
+    // counter of the device-wide fill
+    DevBuf s_dpbig, s_grows, s_growoff, s_fail, s_gstrip0, s_gnext;
     DpBuckets dpb{};
     // a pair is filled by several waves when Lq*Lr >= mw_min_cells and it
     // has at least mw_min_strips 64-row strips (and Lr >= 256)
@@ -281,8 +282,8 @@ static std::vector<DevBuf*> all_bufs(gta_ctx* c) {
             &c->s_flags, &c->s_grand, &c->s_best0, &c->s_prev, &c->s_naln, &c->s_qpos,
             &c->s_rpos, &c->s_fndx, &c->s_fpos, &c->s_tibest, &c->s_tgrand, &c->s_out,
             &c->s_aln, &c->s_btck, &c->s_btckoff, &c->s_rowbuf, &c->s_cells, &c->s_alns,
-            &c->s_algb, &c->s_dpsmall, &c->s_dpbig, &c->s_ring, &c->s_ringoff, &c->s_fail,
-            &c->s_gstrip0, &c->s_gsync,
+            &c->s_algb, &c->s_dpbig, &c->s_grows, &c->s_growoff, &c->s_fail,
+            &c->s_gstrip0, &c->s_gnext,
             &c->s_rsmall, &c->s_rbig, &c->s_parts, &c->s_bigmask, &c->s_lista, &c->s_listb,
             &c->s_listc, &c->s_lcnt, &c->s_ltot, &c->s_heads, &c->s_sctfm, &c->s_scflag,
             &c->s_scout};
@@ -407,64 +408,58 @@ static int ilog2ll(long long v) {
     return r;
 }
 
-// per-pair forms -> device lists [one | W4 | W8 | W16 | grid], ring offsets and
-// strip counters
+// per-pair forms -> device lists [one | W4 | W8 | W16 | grid], and the rows and
+// strip items of the grid pairs
 static int upload_dp_buckets(gta_ctx* c, const std::vector<unsigned char>& form, DpBuckets& B) {
     const int nr = c->r.nstrs;
     const size_t np = form.size();
-    std::vector<int> lists[DPF_N];
-    for (size_t p = 0; p < np; p++) lists[form[p]].push_back((int)p);
     B = DpBuckets{};
     HIPCHK(c, c->s_fail.ensure(4));
     B.failflag = c->s_fail.as<int>();
+    std::vector<int> lists[DPF_N];
+    for (size_t p = 0; p < np; p++) lists[form[p]].push_back((int)p);
     if (lists[DPF_ONE].size() == np) return GTA_OK;     // small == nullptr: every pair one wave
     std::vector<int> all;
-    std::vector<unsigned long long> offs;
     size_t start[DPF_N];
-    unsigned long long ringtot = 0;
     for (int f = 0; f < DPF_N; f++) {
         start[f] = all.size();
-        for (int pidx : lists[f]) {
-            all.push_back(pidx);
-            const int Lq = c->q.len[pidx / nr], Lr = c->r.len[pidx % nr];
-            offs.push_back(ringtot);
-            if (f == DPF_ONE) continue;
-            const unsigned long long rows =
-                f == DPF_GRID ? (unsigned long long)((Lq + 63) / 64) : (4ull << (f - DPF_W4));
-            ringtot += rows * (unsigned long long)Lr;
-        }
+        all.insert(all.end(), lists[f].begin(), lists[f].end());
     }
-    std::vector<int> s0;
-    int tot = 0;
-    for (int pidx : lists[DPF_GRID]) {
-        s0.push_back(tot);
-        tot += (c->q.len[pidx / nr] + 63) / 64;
-    }
-    s0.push_back(tot);
     HIPCHK(c, c->s_dpbig.ensure(all.size() * 4));
-    HIPCHK(c, c->s_ringoff.ensure(offs.size() * 8));
-    HIPCHK(c, c->s_ring.ensure(std::max<unsigned long long>(ringtot, 1) * 4));
-    HIPCHK(c, c->s_gstrip0.ensure(s0.size() * 4));
-    HIPCHK(c, c->s_gsync.ensure(((size_t)tot + 1) * 4));
     HIPCHK(c, hipMemcpy(c->s_dpbig.p, all.data(), all.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->s_ringoff.p, offs.data(), offs.size() * 8, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->s_gstrip0.p, s0.data(), s0.size() * 4, hipMemcpyHostToDevice));
     const int* L = c->s_dpbig.as<int>();
-    const unsigned long long* O = c->s_ringoff.as<unsigned long long>();
     B.small = L + start[DPF_ONE];
     B.nsmall = (int)lists[DPF_ONE].size();
     for (int g = 0; g < 3; g++) {
         B.mw[g] = L + start[DPF_W4 + g];
         B.nmw[g] = (int)lists[DPF_W4 + g].size();
-        B.mwoff[g] = O + start[DPF_W4 + g];
     }
-    B.ring = c->s_ring.as<float>();
     B.grid = L + start[DPF_GRID];
     B.ngrid = (int)lists[DPF_GRID].size();
+    if (B.ngrid == 0) return GTA_OK;
+    std::vector<int> s0;
+    std::vector<unsigned long long> offs;
+    unsigned long long rowtot = 0;
+    int tot = 0;
+    for (int pidx : lists[DPF_GRID]) {
+        const int ns = (c->q.len[pidx / nr] + 63) / 64;
+        s0.push_back(tot);
+        offs.push_back(rowtot);
+        tot += ns;
+        rowtot += (unsigned long long)ns * (unsigned long long)c->r.len[pidx % nr];
+    }
+    s0.push_back(tot);
+    HIPCHK(c, c->s_growoff.ensure(offs.size() * 8));
+    HIPCHK(c, c->s_grows.ensure(rowtot * 4));
+    HIPCHK(c, c->s_gstrip0.ensure(s0.size() * 4));
+    HIPCHK(c, c->s_gnext.ensure(4));
+    HIPCHK(c, hipMemcpy(c->s_growoff.p, offs.data(), offs.size() * 8, hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->s_gstrip0.p, s0.data(), s0.size() * 4, hipMemcpyHostToDevice));
     B.gstrip0 = c->s_gstrip0.as<int>();
-    B.gtotal = tot;
-    B.gsync = c->s_gsync.as<int>();
-    B.growoff = O + start[DPF_GRID];
+    B.gnext = c->s_gnext.as<int>();
+    B.grows = c->s_grows.as<float>();
+    B.growoff = c->s_growoff.as<unsigned long long>();
+    B.growtot = rowtot;
     B.gworkers = std::max(1, std::min(tot, 2 * c->ncu));
     return GTA_OK;
 }

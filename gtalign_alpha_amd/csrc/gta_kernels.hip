@@ -697,15 +697,16 @@ __global__ __launch_bounds__(RTHREADS) void k_refine_gapless(DevChunk Q, DevChun
 }
 
 // ============================================================================
-// DP fill with backtrace and extraction of matched pairs, one wave per pair.
+// DP fill with backtrace and extraction of matched pairs.
 //
-// The Lq x Lr matrix is swept in strips of 64 query rows; lane l owns row
-// 64*s + l and at step t computes column t - l, so every step is one
-// anti-diagonal of the strip.  The up and diagonal predecessors come from lane
-// l-1 through a cross-lane shift; lane 0 takes the previous strip's last row
-// (staged with the reference columns) and lane 63's values leave through a
-// second shift into the row the next strip reads.  Every lane packs its own
-// 2-bit backtrace codes of 16 steps into one word: 64 words, one coalesced
+// The Lq x Lr matrix is swept in strips of 64 R query rows (R = 1..4): lane l
+// owns the R consecutive rows from 64 g0 + l R on (g0: the strip's first group
+// of 64 rows) and at step t computes column t - l of them, so every step is
+// one staircase diagonal of the strip.  The up and diagonal predecessors of a
+// lane's first row come from lane l-1 through a cross-lane shift; lane 0 takes
+// the previous strip's last row and lane 63's last row leaves through a second
+// shift into the row the next strip reads.  Every lane packs its own 2-bit
+// backtrace codes of 16 steps into one word per row: 64 words, one coalesced
 // 256-byte store.  The walk from the bottom-right cell reads runs of 64 cells
 // along the current direction in parallel.
 enum { DPM_IBEST = 0, DPM_GRAND = 1, DPM_CONSTRAINED = 2 };
@@ -748,13 +749,30 @@ __device__ __forceinline__ void load_gtab(float* gtab, float rrw) {
     __syncthreads();
 }
 
-// Backtrace word of lane l in block (s, tb): the codes of row 64s+l at the
-// strip's steps 16tb..16tb+15, step t at bits 2(t&15); cell (i, j) is row i
-// at step t = j + (i & 63).
-__device__ __forceinline__ unsigned read_code(const unsigned* bt, int nblk, int i, int j) {
-    const int s = i >> 6, l = i & 63, t = j + l;
-    const unsigned w = bt[((size_t)(s * nblk + (t >> 4)) << 6) + l];
-    return (w >> ((t & 15) << 1)) & 3u;
+// Rows per lane of a strip: a fill form's strips hold rm groups of 64 rows
+// each, the last one the groups that are left.  One wave per pair takes
+// rm = 4: the ring read, the cross-lane shift, the block bookkeeping and the 63
+// skewed steps are paid once per four rows, and four independent cell scores
+// are in flight.  The forms that run a pair's strips in parallel take rm = 1.
+constexpr int DP_RM = 4;
+// Waves per SIMD that the one-wave kernel is compiled for: 128 registers hold
+// an unrolled block of 8 steps of four rows without spills in it.  DP of a
+// 16 x 12,000 search, 30 fills: 3 waves 110.2 ms, 4 105.6, 5 110.9, 6 120.0,
+// 8 130.7; blocks of 16 steps of every strip 109.7, of strips of one or two
+// rows 105.6, 8 everywhere 102.9.
+constexpr int DP_WAVES = 4;
+
+// Backtrace word of row i at step t = j + lane, lane and k its lane and row
+// within the lane: block (t >> 4) of the strip holds R x 64 words, row k's
+// first at 64 k; step t's code is at bits 2 (t & 15).  A strip's blocks start
+// at 64 nblk words per group of rows above it.  Returns the row's word of
+// block 0; block b's lies 64 b R words on.
+__device__ __forceinline__ const unsigned* code_row(const unsigned* bt, int nblk, int rm, int ngroups, int i, int& R,
+                                                    int& lane) {
+    const int g0 = rm == 1 ? i >> 6 : (i / (64 * rm)) * rm, r = i - (g0 << 6);
+    R = min(rm, ngroups - g0);
+    lane = R == 1 ? r : R == 2 ? r >> 1 : R == 3 ? r / 3 : r >> 2;
+    return bt + ((size_t)(g0 * nblk + (r - lane * R)) << 6) + lane;
 }
 
 // whole-wave shifts by one lane (DPP wave_shr:1 and wave_shl:1): lane l
@@ -812,269 +830,290 @@ __device__ __forceinline__ bool dp_setup(const DevChunk& Q, const DevChunk& R, c
     return true;
 }
 
-// Row handoff between the strips of one wave: nothing to wait for.
-struct NoSync {
-    __device__ __forceinline__ bool wait(int, int) { return true; }
-    __device__ __forceinline__ void publish(int, int) {}
+// The reference columns of one wave's strip in LDS: a ring of DPRING entries
+// {x, y, z, SS letter} (two 64-column blocks; column c at entry c mod DPRING),
+// whose first 16 entries are repeated behind it, so that the 16 entries from
+// any on lie in a row and a block of 16 steps addresses them with immediate
+// offsets; and the 16 values of the row above that lane 0 takes in the block
+// (the value as a left move sees it, and as a diagonal move does).
+constexpr int DPRING = 128;
+struct DpLds {
+    float4 ring[DPRING + 16];
+    float2 up[16];
 };
 
-// LDS staging of one wave's reference columns: a ring of DPRING entries (two
-// 64-column blocks) of {x, y, z, row-above value}, and the SS letters in a
-// float ring of the same size.  Column c lives at entry c mod DPRING.
-constexpr int DPRING = 128;
+// Row handoff of a pair whose strips one wave sweeps in turn: the pair's row
+// in HBM, read a block of 16 steps ahead and overwritten 64 columns behind.
+struct RowMem {
+    static constexpr bool IN_LDS = false;
+    const float* in;
+    float* out;
+    // the value of column c for the next block (lanes 0-15)
+    __device__ __forceinline__ float fetch(int c, int Lr) { return (lane_id() < 16 && c < Lr) ? in[c] : 0.f; }
+    // v: the fetched values of columns t0 + lane; false when a wait gave up
+    __device__ __forceinline__ bool take(float&, int, int) { return true; }
+    // lanes 48-63 hold columns c of the strip's last row
+    __device__ __forceinline__ bool put(int c, int, int Lr, float v) {
+        if (lane_id() >= 48 && c >= 0 && c < Lr) out[c] = v;
+        return true;
+    }
+};
 
-// One strip of 64 query rows of the DP (the strip sweep of every DP kernel).
-// Lane l owns row 64s+l and at step t computes column t-l, so a step advances
-// one anti-diagonal.  Each lane reads its column's entry from the LDS ring
-// (prefetched a step ahead); the whole wave loads the next 64-column block
-// coalesced from HBM a block ahead and writes it into the ring when the block
-// it replaces has been read.  The row above the strip (rowin, written by the
-// previous strip) comes in the same blocks and reaches lane 0 with the
-// up-shift of the values; lane 63's values leave through a down-shift
-// conveyor into rowout, stored and published a block at a time.  No divergent
-// branches in the step loop.  SC is the cell score kind (SC_*); GAP0 fixes
-// the gap mode at compile time; without BTCK no backtrace is written
-// (score-only fills).  vend, when given, receives each lane's value at the
-// strip's last column (row 64s+l).  SC_SSRR ring entries hold {residue code
-// (int bits), SS letter, 0, row-above value} and read the weighted residue
-// scores from gtab.  Returns false when a row wait gave up (Sync::wait).
-// PUT: the strip stores its last row (rowout given), fixed at compile time.
-// The steps where every lane's cell lies inside the matrix (a strip of 64 rows
-// of the query, steps 63 to Lr-1) run a form without the bounds selects.
-template <int SC, bool GAP0, bool BTCK, bool PUT, class Sync>
-__device__ __forceinline__ bool dp_strip_impl(const DevChunk& Q, const DevChunk& R, const DevState& S,
-                                              const DpParams& prm, const DpPair& P, int s, const float* rowin,
-                                              float* rowout, unsigned* bt, float4* ring, float* ssring,
-                                              Sync& sync, float* vend, const float* gtab) {
+// One strip of R x 64 query rows of the DP (the sweep of every DP kernel),
+// from group g0 on.  The whole wave loads the next 64 reference columns
+// coalesced from HBM a block ahead and writes them into the LDS ring when the
+// block they replace has been read.  The steps run in blocks of 16, 8 of them
+// unrolled: ring offsets and code shifts are then immediates, no value is
+// copied between steps, and bounds, row handoff and stores are looked at once
+// a block.  A block holding a lane left of the
+// matrix or undefined coordinates runs a form that zeroes those cells' scores
+// (the columns before the first one are undefined entries, so their cells stay
+// 0); every other block runs without any select on the score.  Cells past the
+// last column or row are computed and never read.
+// SC is the cell score kind (SC_*); GAP0 fixes the gap mode at compile time;
+// without BTCK no backtrace is written (score-only fills), and vend receives
+// the values of the lane's rows at the last column.  SC_SSRR ring entries hold
+// {residue code (int bits), SS letter} and read the weighted residue scores
+// from gtab.  Below a strip (g0 > 0) the row above comes through io; PUT: this
+// strip hands its own last row over.  Returns false when a row wait gave up.
+//
+// Bound by VALU issue: 22 instructions a cell in the inner blocks of the
+// distance score without gap cost (16 full-rate ones and the quarter-rate
+// reciprocal for the score and the sum, 5.5 half-rate ones for the maximum and
+// the code), against 29 with one row a lane and rolled steps.  Fill alone of
+// 16,384 pairs of 1,024 x 1,024: 1,176 -> 1,660 G cells/s; 40,000 pairs of
+// 256 x 256 with the walk 3.18 -> 2.27 ms (with SS letters and gap cost
+// 3.99 -> 2.77 ms).
+template <int SC, bool GAP0, bool BTCK, int R, bool PUT, class IO>
+__device__ __forceinline__ bool dp_sweep(const DevChunk& Q, const DevChunk& Rf, const DpParams& prm,
+                                         const DpPair& P, int g0, unsigned* bt, DpLds& lds, IO& io, float* vend,
+                                         const float* gtab) {
     constexpr bool USESS = SC == SC_TMSS;
     constexpr bool SSRR = SC == SC_SSRR;
+    constexpr int U = 8;            // steps per unrolled block, two to a code word
     // value of the cells outside the matrix
     constexpr float OUT = SSRR ? DPSS_INIT : 0.0f;
+    // an entry outside the matrix: undefined, with an SS letter nothing matches
+    const float4 outside = make_float4(SSRR ? 0.f : 2.f * DEFCOORD_RFN_cmp, 0.f, 0.f, -1.f);
     const int lane = lane_id();
     const int Lq = P.Lq, Lr = P.Lr;
-    const float* Rx = R.x + P.rd;
-    const float* Ry = R.y + P.rd;
-    const float* Rz = R.z + P.rd;
-    const char* Rs = R.ss + P.rd;
-    const char* Rr = R.rsd + P.rd;
     const float gapopen = prm.gapopen, ssw = prm.ssw, d02 = P.d02;
-    const int nsteps = Lr + 63;
-    const int nblkw = (nsteps + 15) >> 4;
-    const int i = (s << 6) + lane;
-    const bool rowok = i < Lq;
-    float qx = 0.f, qy = 0.f, qz = 0.f;
-    float qss = 0.f;
-    int qbase = 0;      // SC_SSRR: the lane's row of gtab
-    if (rowok) {
-        if (SSRR) {
-            qss = (float)Q.ss[P.qd + i];
-            qbase = res_code(Q.rsd[P.qd + i]) * NGT;
-        } else {
-            qx = Q.x[P.qd + i]; qy = Q.y[P.qd + i]; qz = Q.z[P.qd + i];
-            tfm_point(P.tfm, qx, qy, qz);
-            if (USESS) qss = (float)Q.ss[P.qd + i];
-        }
-    }
-    const bool qok = rowok && qx < DEFCOORD_QRY_cmp;
-    const bool haveup = rowin != nullptr;
-    constexpr bool putrow = PUT;
-    if (haveup && !sync.wait(s - 1, min(128, Lr))) return false;
-    // block 0 at entries 0..63, columns -64..-1 (entries 64..127) outside
-    {
-        const int c = lane;
-        const bool ok = c < Lr;
-        if (SSRR)
-            ring[lane] = make_float4(__int_as_float(ok ? res_code(Rr[c]) : 0), ok ? (float)Rs[c] : 0.f, 0.f,
-                                     (ok && haveup) ? rowin[c] : OUT);
-        else
-            ring[lane] = make_float4(ok ? Rx[c] : 0.f, ok ? Ry[c] : 0.f, ok ? Rz[c] : 0.f,
-                                     (ok && haveup) ? rowin[c] : OUT);
-        ring[64 + lane] = make_float4(0.f, 0.f, 0.f, OUT);
-        if (USESS) {
-            ssring[lane] = ok ? (float)Rs[c] : 0.f;
-            ssring[64 + lane] = 0.f;
-        }
-    }
-    // the next block waits in registers
-    float nbx, nby, nbz, nbu, nbs = 0.f;
-    {
-        const int c2 = 64 + lane;
-        const bool ok2 = c2 < Lr;
-        if (SSRR) {
-            nbx = __int_as_float(ok2 ? res_code(Rr[c2]) : 0); nby = ok2 ? (float)Rs[c2] : 0.f; nbz = 0.f;
-        } else {
-            nbx = ok2 ? Rx[c2] : 0.f; nby = ok2 ? Ry[c2] : 0.f; nbz = ok2 ? Rz[c2] : 0.f;
-        }
-        if (USESS) nbs = ok2 ? (float)Rs[c2] : 0.f;
-        nbu = (ok2 && haveup) ? rowin[c2] : OUT;
-    }
-    int ao = ((-lane) & (DPRING - 1)) << 4;  // byte offset of column t - lane's ring entry
-    float4 cur = *(const float4*)((const char*)ring + ao);
-    float curs = USESS ? ssring[ao >> 4] : 0.f;
-    float val = OUT, upprev = OUT, oblk = 0.f;
-    unsigned word = 0;
-    int j = -lane;
-    // one step (anti-diagonal); false when a row wait gave up.  In an inner
-    // step every lane's cell is in the matrix, so the bounds test (and the
-    // column counter it reads) drops out.
-    auto step = [&](const int t, auto kind) -> bool {
-        // kind 0: edge step; 1: inner step; 2: inner step of a strip whose
-        // query rows and reference columns all hold defined coordinates
-        constexpr bool INNER = decltype(kind)::value >= 1;
-        constexpr bool DEFINED = decltype(kind)::value == 2;
-        const float4 rc = cur;
-        const float rss = curs;
-        if ((t & 63) == 63) {
-            // block (t+1)/64 replaces columns t-127..t-64, all read by now
-            const int e = (t + 1 + lane) & (DPRING - 1);
-            ring[e] = make_float4(nbx, nby, nbz, nbu);
-            if (USESS) ssring[e] = nbs;
-            const int c2 = t + 65 + lane;
-            const bool ok2 = c2 < Lr;
-            if (SSRR) {
-                nbx = __int_as_float(ok2 ? res_code(Rr[c2]) : 0); nby = ok2 ? (float)Rs[c2] : 0.f;
-            } else {
-                nbx = ok2 ? Rx[c2] : 0.f; nby = ok2 ? Ry[c2] : 0.f; nbz = ok2 ? Rz[c2] : 0.f;
-            }
-            if (USESS) nbs = ok2 ? (float)Rs[c2] : 0.f;
-            if (haveup && t + 65 < Lr) {
-                if (!sync.wait(s - 1, min(t + 129, Lr))) return false;
-            }
-            nbu = (ok2 && haveup) ? rowin[c2] : OUT;
-        }
-        ao = (ao + 16) & (DPRING * 16 - 1);
-        cur = *(const float4*)((const char*)ring + ao);
-        if (USESS) curs = ssring[ao >> 4];
+    const float* Rx = Rf.x + P.rd;
+    const float* Ry = Rf.y + P.rd;
+    const float* Rz = Rf.z + P.rd;
+    const char* Rs = Rf.ss + P.rd;
+    const char* Rr = Rf.rsd + P.rd;
 
-        const float up = wave_shr1(val, rc.w);
-        const float diag = upprev;
-        upprev = up;
-        const bool valid = INNER || (rowok && (unsigned)j < (unsigned)Lr);
-        float v, nv;
-        unsigned bk = BT_DIAG;
+    float qx[R], qy[R], qz[R], qss[R];
+    int qbase[R];       // SC_SSRR: the row's line of gtab
+    bool qok[R], alldef = true;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        // rows past the last one take its coordinates (their cells are never
+        // read): the loads of all rows are issued at once
+        const int i = min((g0 << 6) + lane * R + k, Lq - 1);
+        qx[k] = qy[k] = qz[k] = qss[k] = 0.f;
+        qbase[k] = 0;
         if (SSRR) {
-            // (float)(SS match) * wss + residue score * wrr, then the shifted
-            // recurrence (MpDPHub.cpp:1150-1185)
-            float sc = __fmul_rn(qss == rc.y ? 1.0f : 0.0f, ssw);
-            sc = __fadd_rn(sc, gtab[qbase + __float_as_int(rc.x)]);
-            float d = diag;
-            if (d < DPSS_INIT_cmp) d = __fsub_rn(d, DPSS_INIT);
-            v = __fadd_rn(sc, d);
-            float w = val;
-            if (w < DPSS_INIT_cmp) w = __fsub_rn(__fadd_rn(gapopen, w), DPSS_INIT);
-            if (v < w) { v = w; bk = BT_LEFT; }
-            w = up;
-            if (w < DPSS_INIT_cmp) w = __fsub_rn(__fadd_rn(gapopen, w), DPSS_INIT);
-            if (v < w) { v = w; bk = BT_UP; }
-            nv = (bk != BT_DIAG) ? v : __fadd_rn(v, DPSS_INIT);
+            qss[k] = (float)Q.ss[P.qd + i];
+            qbase[k] = res_code(Q.rsd[P.qd + i]) * NGT;
         } else {
-            float sc = pair_score(d02, dist2(qx, qy, qz, rc.x, rc.y, rc.z));
-            if (!DEFINED) sc = (qok && DEFCOORD_RFN_cmp < rc.x) ? sc : 0.0f;
-            if (USESS) sc = __fadd_rn(sc, (qss == rss) ? ssw : 0.0f);
-            v = __fadd_rn(sc, GAP0 ? diag : fabsf(diag));
-            float w = val;
-            if (!GAP0 && w < 0.0f) w = __fsub_rn(gapopen, w);
-            if (v < w) { v = w; bk = BT_LEFT; }
-            w = up;
-            if (!GAP0 && w < 0.0f) w = __fsub_rn(gapopen, w);
-            if (v < w) { v = w; bk = BT_UP; }
-            nv = (GAP0 || bk != BT_DIAG) ? v : -v;
+            qx[k] = Q.x[P.qd + i]; qy[k] = Q.y[P.qd + i]; qz[k] = Q.z[P.qd + i];
+            if (USESS) qss[k] = (float)Q.ss[P.qd + i];
         }
-        // cells left of the strip's columns keep 0, cells past them the last value
-        val = valid ? nv : val;
-        const unsigned code = valid ? bk : (unsigned)BT_STOP;
-        if (!INNER) j++;
-        if (putrow) {
-            // lane l now holds column t-126+l of row 64s+63
-            oblk = wave_shl1(oblk, val);
-            const int jo = t - 63;
-            if (jo >= 0 && ((jo & 63) == 63 || jo == Lr - 1)) {
-                if (lane >= 63 - (jo & 63)) rowout[jo - 63 + lane] = oblk;
-                sync.publish(s, jo + 1);
-            }
+    }
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        if (!SSRR) tfm_point(P.tfm, qx[k], qy[k], qz[k]);
+        qok[k] = qx[k] < DEFCOORD_QRY_cmp;
+        alldef &= qok[k];
+    }
+    // entry of column c (past the last column: the last one's, never used)
+    auto entry = [&](int c) -> float4 {
+        const int o = min(c, Lr - 1);
+        if (SSRR) return make_float4(__int_as_float(res_code(Rr[o])), (float)Rs[o], 0.f, 0.f);
+        return make_float4(Coords::at(Rx, o), Coords::at(Ry, o), Coords::at(Rz, o), USESS ? (float)Rs[o] : 0.f);
+    };
+    auto undefined = [&](const float4& e) { return !SSRR && __any(!(DEFCOORD_RFN_cmp < e.x)); };
+    float4 nb = entry(lane);
+    // blocks from t0 <= gen on run the general form: lanes left of the matrix
+    // until step 62, and the 127 steps that see a 64-column block with an
+    // undefined entry
+    int gen = (!SSRR && !__all(alldef)) ? 0x7fffffff : undefined(nb) ? 126 : 62;
+    lds.ring[lane] = nb;
+    if (lane < 16) lds.ring[DPRING + lane] = nb;
+    lds.ring[64 + lane] = outside;
+    const bool haveup = g0 > 0;
+    if (!haveup && lane < 16) lds.up[lane] = make_float2(OUT, OUT);
+    nb = entry(64 + lane);
+
+    const int nsteps = Lr + 63, nblk = (nsteps + 15) >> 4;
+    // the row's values in the lane's current column: GAP0 and SC_SSRR keep the
+    // value; with a gap cost a cell reached diagonally costs gapopen to leave
+    // sideways, so val is what the neighbours below and to the right compare
+    // (the value, or gapopen more), mag what a diagonal move adds to
+    float val[R], mag[R];
+    float upprev = OUT, oblk = 0.f, pre = 0.f;
+    unsigned word[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) { val[k] = mag[k] = OUT; word[k] = 0; }
+    // the row above for the 16 columns from t on, and the load of the next 16
+    auto above = [&](int t) -> bool {
+        if (!io.take(pre, t, Lr)) return false;
+        if (lane < 16) {
+            // a stored value < 0 was reached diagonally
+            if (GAP0 || SSRR) lds.up[lane] = make_float2(pre, pre);
+            else lds.up[lane] = make_float2(pre < 0.f ? __fsub_rn(gapopen, pre) : pre, fabsf(pre));
         }
-        if (BTCK) {
-            word |= code << ((t & 15) << 1);
-            if ((t & 15) == 15 || t == nsteps - 1) {
-                bt[((size_t)(s * nblkw + (t >> 4)) << 6) + lane] = word;
-                word = 0;
-            }
-        }
+        pre = io.fetch(t + 16 + lane, Lr);
         return true;
     };
-    // two steps per iteration, so that the prefetched ring entry and the
-    // carried values alternate registers instead of being copied every step
-    const std::integral_constant<int, 0> edge;
-    const std::integral_constant<int, 1> inner;
-    const std::integral_constant<int, 2> inner_defined;
-    // inner steps: a full strip, steps 64 .. (Lr & ~1) - 1 (even bounds keep the pairs)
-    const bool full = (s + 1) << 6 <= Lq;
-    const int tin = full ? 64 : nsteps, tout = full ? max(64, Lr & ~1) : nsteps;
-    // a full strip whose 64 query rows and Lr reference columns are all
-    // defined scores every inner cell without the undefined-coordinate select
-    // (the select would keep the score in every such cell).  The check reads
-    // the reference's x once per strip (independent loads, no early exit);
-    // references longer than 4,096 residues, whose strips the device-wide
-    // pipeline runs back to back, keep the select instead.
-    bool defined = false;
-    if (!SSRR && full && Lr <= 4096) {
-        bool d = qok;
-#pragma unroll 4
-        for (int c = lane; c < Lr; c += GTA_WAVE) d &= DEFCOORD_RFN_cmp < Rx[c];
-        defined = __all(d);
+    if (haveup) {
+        pre = io.fetch(lane, Lr);
+        if (!above(0)) return false;
     }
-    int t = 0;
-    for (; t + 1 < min(tin, nsteps); t += 2) {
-        if (!step(t, edge)) return false;
-        if (!step(t + 1, edge)) return false;
-    }
-    if (t < tout) {
-        if (defined) {
-            for (; t + 1 < tout; t += 2) {
-                if (!step(t, inner_defined)) return false;
-                if (!step(t + 1, inner_defined)) return false;
+
+    for (int b = 0; b < nblk; b++) {
+        const int t0 = b << 4;
+        __builtin_amdgcn_wave_barrier();
+        auto block = [&](auto kind) {
+            constexpr bool GEN = decltype(kind)::value;
+#pragma unroll 1
+            for (int h = 0; h < 16; h += U) {
+                const float4* rp = lds.ring + ((t0 + h - lane) & (DPRING - 1));
+                const float2* upp = lds.up + h;
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const float4 rc = rp[u];
+                    const float2 fill = upp[u];
+                    float up = wave_shr1(val[R - 1], fill.x);
+                    float dg = upprev;
+                    upprev = (GAP0 || SSRR) ? up : wave_shr1(mag[R - 1], fill.y);
+                    float sgn = 0.f;
+#pragma unroll
+                    for (int k = 0; k < R; k++) {
+                        unsigned code;
+                        if (SSRR) {
+                            // (float)(SS match) * wss + residue score * wrr, then the
+                            // shifted recurrence (MpDPHub.cpp:1150-1185)
+                            float sc = __fmul_rn(qss[k] == rc.y ? 1.0f : 0.0f, ssw);
+                            sc = __fadd_rn(sc, gtab[qbase[k] + __float_as_int(rc.x)]);
+                            float d = dg;
+                            if (d < DPSS_INIT_cmp) d = __fsub_rn(d, DPSS_INIT);
+                            float v = __fadd_rn(sc, d);
+                            code = BT_DIAG;
+                            float w = val[k];
+                            if (w < DPSS_INIT_cmp) w = __fsub_rn(__fadd_rn(gapopen, w), DPSS_INIT);
+                            if (v < w) { v = w; code = BT_LEFT; }
+                            w = up;
+                            if (w < DPSS_INIT_cmp) w = __fsub_rn(__fadd_rn(gapopen, w), DPSS_INIT);
+                            if (v < w) { v = w; code = BT_UP; }
+                            if (code == BT_DIAG) v = __fadd_rn(v, DPSS_INIT);
+                            dg = val[k];
+                            val[k] = (GEN && t0 + h + u < lane) ? OUT : v;
+                            up = val[k];
+                            sgn = val[k];
+                        } else {
+                            float sc = pair_score(d02, dist2(qx[k], qy[k], qz[k], rc.x, rc.y, rc.z));
+                            if (GEN) sc = (qok[k] && DEFCOORD_RFN_cmp < rc.x) ? sc : 0.0f;
+                            if (USESS) sc = __fadd_rn(sc, (qss[k] == rc.w) ? ssw : 0.0f);
+                            const float v = __fadd_rn(sc, dg), w = val[k];
+                            // DIAG unless a neighbour is better, LEFT unless the one above is better still
+                            if (GAP0) {
+                                const float nv = fmaxf(fmaxf(v, w), up);
+                                code = (v < nv) ? (w < up ? BT_UP : BT_LEFT) : BT_DIAG;
+                                dg = w;
+                                val[k] = up = sgn = nv;
+                            } else {
+                                const float m = fmaxf(w, up);
+                                const bool side = v < m;
+                                code = side ? (w < up ? BT_UP : BT_LEFT) : BT_DIAG;
+                                dg = mag[k];
+                                mag[k] = fmaxf(v, m);
+                                // a defined cell's score is positive, and with it v; an undefined
+                                // one's may be 0, which leaves it sideways at no cost
+                                const float open = (!GEN || 0.0f < v) ? __fadd_rn(gapopen, v) : v;
+                                val[k] = up = side ? m : open;
+                                sgn = side ? m : -v;
+                            }
+                        }
+                        if (BTCK) word[k] |= code << (2 * u + 16);
+                        if (!BTCK && t0 + h + u - lane == Lr - 1) vend[k] = sgn;
+                    }
+                    // lane l now holds column t-126+l of the strip's last row
+                    if (PUT) oblk = wave_shl1(oblk, sgn);
+                }
+                if (BTCK && h == 0) {
+#pragma unroll
+                    for (int k = 0; k < R; k++) word[k] >>= 16;
+                }
             }
-        } else {
-            for (; t + 1 < tout; t += 2) {
-                if (!step(t, inner)) return false;
-                if (!step(t + 1, inner)) return false;
+        };
+        if (t0 <= gen) block(std::true_type{});
+        else block(std::false_type{});
+        // What the next block needs is taken before this block's stores are
+        // issued: a wait for a load also waits for every store before it, and
+        // the ones before these loads are then a block old.  (Behind the
+        // stores, the waits for their acknowledgement held a wave 40% of its
+        // time and the fill of 40,000 pairs of 256 x 256 took 2.27 ms.)
+        const int t1 = t0 + 16;
+        if (PUT && IO::IN_LDS && !io.put(t0 - 111 + lane, t0 - 47, Lr, oblk)) return false;
+        if ((t1 & 63) == 0) {
+            // columns t1..t1+63 replace t1-128..t1-65, all read by now
+            lds.ring[(t1 & (DPRING - 1)) + lane] = nb;
+            if ((t1 & (DPRING - 1)) == 0 && lane < 16) lds.ring[DPRING + lane] = nb;
+            if (undefined(nb)) gen = max(gen, t1 + 126);
+            nb = entry(t1 + 64 + lane);
+        }
+        if (haveup && t1 < Lr && !above(t1)) return false;
+        if (BTCK) {
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                bt[((size_t)(b * R + k) << 6) + lane] = word[k];
+                word[k] = 0;
             }
         }
-        j = t - lane;   // the column counter as the edge steps would have left it
+        if (PUT && !IO::IN_LDS && !io.put(t0 - 111 + lane, t0 - 47, Lr, oblk)) return false;
     }
-    for (; t + 1 < nsteps; t += 2) {
-        if (!step(t, edge)) return false;
-        if (!step(t + 1, edge)) return false;
-    }
-    if (t < nsteps && !step(t, edge)) return false;
-    if (vend) *vend = val;
     return true;
 }
-template <int SC, bool GAP0, bool BTCK = true, class Sync>
-__device__ __forceinline__ bool dp_strip(const DevChunk& Q, const DevChunk& R, const DevState& S,
-                                         const DpParams& prm, const DpPair& P, int s, const float* rowin,
-                                         float* rowout, unsigned* bt, float4* ring, float* ssring, Sync& sync,
-                                         float* vend = nullptr, const float* gtab = nullptr) {
-    if (rowout)
-        return dp_strip_impl<SC, GAP0, BTCK, true>(Q, R, S, prm, P, s, rowin, rowout, bt, ring, ssring, sync,
-                                                   vend, gtab);
-    return dp_strip_impl<SC, GAP0, BTCK, false>(Q, R, S, prm, P, s, rowin, rowout, bt, ring, ssring, sync, vend,
-                                                gtab);
+
+// The strip of `groups` row groups (1..DP_RM) from group g0 on; only strips of
+// DP_RM groups have another below.
+template <int SC, bool GAP0, bool BTCK, class IO>
+__device__ __forceinline__ bool dp_strip(const DevChunk& Q, const DevChunk& R, const DpParams& prm, const DpPair& P,
+                                         int g0, int groups, bool put, unsigned* bt, DpLds& lds, IO& io, float* vend,
+                                         const float* gtab) {
+    if (put) return dp_sweep<SC, GAP0, BTCK, DP_RM, true>(Q, R, prm, P, g0, bt, lds, io, vend, gtab);
+    switch (groups) {
+        case 1: return dp_sweep<SC, GAP0, BTCK, 1, false>(Q, R, prm, P, g0, bt, lds, io, vend, gtab);
+        case 2: return dp_sweep<SC, GAP0, BTCK, 2, false>(Q, R, prm, P, g0, bt, lds, io, vend, gtab);
+        case 3: return dp_sweep<SC, GAP0, BTCK, 3, false>(Q, R, prm, P, g0, bt, lds, io, vend, gtab);
+        default: return dp_sweep<SC, GAP0, BTCK, DP_RM, false>(Q, R, prm, P, g0, bt, lds, io, vend, gtab);
+    }
 }
 
 // Backtrace walk from the bottom-right cell (BtckToMatched, btck2match.cuh:46-52;
-// ConstrainedBtckToMatched keeps pairs within d8 and their d2).  Vectorised:
-// the 64 lanes read 64 successive cells of the current direction and a ballot
-// finds the run length.  Matched pairs are stored in walk (reverse) order.
+// ConstrainedBtckToMatched keeps pairs within d8 and their d2).  Matched pairs
+// are stored in walk (reverse) order.
+//
+// The walk goes through windows of 64 rows: lane l holds the codes of row
+// y0 - l in the 64 columns around the diagonal through the window's first
+// cell (x0 - l - 31 to x0 - l + 32, field f), loaded at once (5 words a lane).
+// A diagonal move keeps f, a move left lowers it, a move up raises it, so a run
+// of diagonal moves is one ballot over the window and every other move one
+// lane's code; no memory access stands between two moves.  A window ends
+// with its rows or when the path leaves its columns.  With one memory access
+// per change of direction the walk took about as long as the fill.
 __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S, const DpParams& prm,
-                        const DpPair& P, const unsigned* bt) {
+                        const DpPair& P, const unsigned* bt, int rm) {
     const int lane = lane_id();
     const int p = P.p, Lq = P.Lq, Lr = P.Lr, qd = P.qd, rd = P.rd;
     if (prm.mode == DPM_GRAND && (P.flags & CONV_SCOREDP)) {
         if (lane == 0) S.nalnposs[p] = 0;
         return;
     }
-    const int nblk = (Lr + 63 + 15) >> 4;
+    const int nblk = (Lr + 63 + 15) >> 4, ngroups = (Lq + 63) >> 6;
     const size_t base = (size_t)P.qi * (size_t)R.nposs + (size_t)rd;
     float* aqx = S.aln + base;
     float* aqy = aqx + S.alnplane;
@@ -1087,46 +1126,64 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
     float* arp = aqp + S.alnplane;
     const bool constrained = prm.mode == DPM_CONSTRAINED;
     const float d82 = GetD82(Lq, Lr);
-    int y = Lq - 1, x = Lr - 1, k = 0;
-    unsigned dir = BT_DIAG;
-    while (y >= 0 && x >= 0) {
-        const int dy = (dir == BT_LEFT) ? 0 : 1, dx = (dir == BT_UP) ? 0 : 1;
-        const int yy = y - lane * dy, xx = x - lane * dx;
-        const bool inr = yy >= 0 && xx >= 0;
-        const unsigned code = inr ? read_code(bt, nblk, yy, xx) : (unsigned)BT_STOP;
-        const unsigned long long brk = __ballot(!(inr && code == dir));
-        const int run = brk ? (int)__builtin_ctzll(brk) : GTA_WAVE;
-        if (dir == BT_DIAG) {
-            const bool take = lane < run;
-            float qx = 0, qy = 0, qz = 0, rx = 0, ry = 0, rz = 0, d2 = 0;
-            bool keep = take;
-            if (take) {
-                qx = Q.x[qd + yy]; qy = Q.y[qd + yy]; qz = Q.z[qd + yy];
-                rx = R.x[rd + xx]; ry = R.y[rd + xx]; rz = R.z[rd + xx];
-                if (constrained) {
-                    d2 = tfm_dist2(P.tfm, qx, qy, qz, rx, ry, rz);
-                    keep = d2 <= d82;
-                }
-            }
-            const unsigned long long km = __ballot(keep);
-            const int before = __popcll(km & ((1ull << lane) - 1ull));
-            if (keep) {
-                const int o = k + before;
-                aqx[o] = qx; aqy[o] = qy; aqz[o] = qz;
-                arx[o] = rx; ary[o] = ry; arz[o] = rz;
-                aqp[o] = (float)yy; arp[o] = (float)xx;
-                if (constrained) ad2[o] = d2;
-            }
-            k += __popcll(km);
+    int y0 = Lq - 1, x0 = Lr - 1, k = 0;
+    while (y0 >= 0 && x0 >= 0) {
+        const int yy = y0 - lane;
+        unsigned c0, c1, c2, c3;    // the codes of fields 0-15, 16-31, 32-47, 48-63
+        {
+            int rows, ln;
+            const unsigned* w = code_row(bt, nblk, rm, ngroups, max(yy, 0), rows, ln);
+            const int t = x0 - lane - 31 + ln, tb = t >> 4;     // step of field 0
+            unsigned v[5];
+#pragma unroll
+            for (int i = 0; i < 5; i++) v[i] = w[(size_t)(min(max(tb + i, 0), nblk - 1) * rows) << 6];
+            const unsigned sh = (unsigned)(t & 15) << 1;
+            c0 = __builtin_amdgcn_alignbit(v[1], v[0], sh);
+            c1 = __builtin_amdgcn_alignbit(v[2], v[1], sh);
+            c2 = __builtin_amdgcn_alignbit(v[3], v[2], sh);
+            c3 = __builtin_amdgcn_alignbit(v[4], v[3], sh);
         }
-        y -= run * dy;
-        x -= run * dx;
-        if (run < GTA_WAVE) {
-            const unsigned c = __shfl(code, run, GTA_WAVE);
-            const int in = __shfl((int)inr, run, GTA_WAVE);
-            if (!in || c == BT_STOP) break;
-            dir = c;
+        int l = 0, f = 31, xm = -1;     // xm: the lane's matched column
+        for (;;) {
+            const unsigned c = f < 32 ? (f < 16 ? c0 : c1) : (f < 48 ? c2 : c3);
+            // cells left of or above the matrix end the walk
+            const int col = x0 - lane - 31 + f;
+            const unsigned code = (yy >= 0 && col >= 0) ? (c >> ((f & 15) << 1)) & 3u : (unsigned)BT_STOP;
+            const unsigned long long diag = __ballot(code == BT_DIAG) >> l;
+            if (diag & 1ull) {
+                const int run = ~diag ? (int)__builtin_ctzll(~diag) : GTA_WAVE;     // at most 64 - l
+                if (lane >= l && lane < l + run) xm = col;
+                l += run;
+            } else {
+                const unsigned here = __builtin_amdgcn_readlane(code, l);
+                if (here == BT_UP) { l++; f++; }
+                else if (here == BT_LEFT) f--;
+                else { l = -1; break; }
+            }
+            if (l >= GTA_WAVE || f < 0 || f > 63) break;
         }
+        float qx = 0, qy = 0, qz = 0, rx = 0, ry = 0, rz = 0, d2 = 0;
+        bool keep = xm >= 0;
+        if (keep) {
+            qx = Q.x[qd + yy]; qy = Q.y[qd + yy]; qz = Q.z[qd + yy];
+            rx = R.x[rd + xm]; ry = R.y[rd + xm]; rz = R.z[rd + xm];
+            if (constrained) {
+                d2 = tfm_dist2(P.tfm, qx, qy, qz, rx, ry, rz);
+                keep = d2 <= d82;
+            }
+        }
+        const unsigned long long km = __ballot(keep);
+        if (keep) {
+            const int o = k + __popcll(km & ((1ull << lane) - 1ull));
+            aqx[o] = qx; aqy[o] = qy; aqz[o] = qz;
+            arx[o] = rx; ary[o] = ry; arz[o] = rz;
+            aqp[o] = (float)yy; arp[o] = (float)xm;
+            if (constrained) ad2[o] = d2;
+        }
+        k += __popcll(km);
+        if (l < 0) break;
+        y0 -= l;
+        x0 += f - 31 - l;
     }
     if (lane == 0) S.nalnposs[p] = k;
 }
@@ -1147,42 +1204,41 @@ __device__ __forceinline__ void dp_count(const DevState& S, const DpPair& P) {
 // maps blocks to pairs).  The strips run in order; each reads the row the
 // previous one wrote to the pair's row in HBM.
 template <int SC, bool GAP0>
-__device__ void dp_pair(const DevChunk& Q, const DevChunk& R, const DevState& S, const DpParams& prm, int p,
-                        float4* ring, float* ssring, const float* gtab) {
+__device__ __forceinline__ void dp_pair(const DevChunk& Q, const DevChunk& R, const DevState& S, const DpParams& prm, int p,
+                        DpLds& lds, const float* gtab) {
     DpPair P;
     if (!dp_setup(Q, R, S, prm, p, P)) return;
     float* row = S.rowbuf + (size_t)P.qi * (size_t)R.nposs + (size_t)P.rd;
     unsigned* bt = S.btck + S.btckoff[P.p];
-    const int nstrips = (P.Lq + 63) >> 6;
-    NoSync ns;
-    for (int s = 0; s < nstrips; s++) {
-        dp_strip<SC, GAP0>(Q, R, S, prm, P, s, s > 0 ? row : nullptr, s + 1 < nstrips ? row : nullptr, bt, ring,
-                           ssring, ns, nullptr, gtab);
+    const int ngroups = (P.Lq + 63) >> 6, nblk = (P.Lr + 63 + 15) >> 4;
+    RowMem io{row, row};
+    for (int g0 = 0; g0 < ngroups; g0 += DP_RM) {
+        dp_strip<SC, GAP0, true>(Q, R, prm, P, g0, min(DP_RM, ngroups - g0), g0 + DP_RM < ngroups,
+                                 bt + ((size_t)(g0 * nblk) << 6), lds, io, nullptr, gtab);
         // the next strip reads this strip's row back
         __threadfence_block();
     }
     dp_count(S, P);
     __threadfence();
-    dp_walk(Q, R, S, prm, P, bt);
+    dp_walk(Q, R, S, prm, P, bt, DP_RM);
 }
 
 // One wave per pair: block b takes pair plist[b] (b without a list), or, with
 // a work queue, the waves of a persistent grid take queued pairs until the
 // queue is drained.
 template <int SC, bool GAP0>
-__global__ __launch_bounds__(GTA_WAVE) __attribute__((amdgpu_waves_per_eu(SC == SC_TMSS ? 6 : 7))) void k_dp(
-    DevChunk Q, DevChunk R, DevState S, DpParams prm,
-                                                  const int* plist, WorkQ wq) {
-    __shared__ float4 ring[DPRING];
-    __shared__ float ssring[SC == SC_TMSS ? DPRING : 1];
+__global__ __launch_bounds__(GTA_WAVE) __attribute__((amdgpu_waves_per_eu(DP_WAVES))) void k_dp(
+    DevChunk Q, DevChunk R, DevState S, DpParams prm, const int* plist, WorkQ wq) {
+    __shared__ DpLds lds;
     __shared__ float gtab[SC == SC_SSRR ? NGT * NGT : 1];
     if (SC == SC_SSRR) load_gtab(gtab, prm.rrw);
-    if (wq.items) {
-        const int n = *wq.count;
-        for (int it = wq_next_wave(wq); it < n; it = wq_next_wave(wq))
-            dp_pair<SC, GAP0>(Q, R, S, prm, wq.items[it], ring, ssring, gtab);
-    } else {
-        dp_pair<SC, GAP0>(Q, R, S, prm, plist ? plist[blockIdx.x] : (int)blockIdx.x, ring, ssring, gtab);
+    const int n = wq.items ? *wq.count : 0;
+    int it = wq.items ? wq_next_wave(wq) : -1;
+    while (it < n) {
+        dp_pair<SC, GAP0>(Q, R, S, prm, wq.items ? wq.items[it] : plist ? plist[blockIdx.x] : (int)blockIdx.x, lds,
+                          gtab);
+        if (!wq.items) break;
+        it = wq_next_wave(wq);
     }
 }
 
@@ -1199,8 +1255,7 @@ template <bool GAP0>
 __global__ __launch_bounds__(GTA_WAVE) void k_dp_score(DevChunk Q, DevChunk R, DevState S, float gapopen,
                                                         const float* tfms, const int* slotflags, int nslots,
                                                         float* scores) {
-    __shared__ float4 ring[DPRING];
-    __shared__ float ssring[1];
+    __shared__ DpLds lds;
     const int np = S.nq * S.nr;
     const int p = blockIdx.x;
     DpPair P;
@@ -1216,9 +1271,8 @@ __global__ __launch_bounds__(GTA_WAVE) void k_dp_score(DevChunk Q, DevChunk R, D
     P.d02 = d0 * d0;
     const DpParams prm{DPM_GRAND, GAP0 ? 1 : 0, gapopen, SC_TM, 0.f, 0, 0.f};
     float* row = S.rowbuf + (size_t)P.qi * (size_t)R.nposs + (size_t)P.rd;
-    const int nstrips = (P.Lq + 63) >> 6;
-    const int lastlane = (P.Lq - 1) & 63;
-    NoSync ns;
+    const int ngroups = (P.Lq + 63) >> 6;
+    RowMem io{row, row};
     for (int k = 0; k < nslots; k++) {
         const size_t o = (size_t)k * np + p;
         if ((P.flags & CONV_LOWTMSC) || (slotflags && slotflags[o])) {
@@ -1227,87 +1281,137 @@ __global__ __launch_bounds__(GTA_WAVE) void k_dp_score(DevChunk Q, DevChunk R, D
         }
 #pragma unroll
         for (int i = 0; i < 12; i++) P.tfm[i] = tfms[o * 12 + i];
-        float vend = 0.f;
-        for (int s = 0; s < nstrips; s++) {
-            dp_strip<SC_TM, GAP0, false>(Q, R, S, prm, P, s, s > 0 ? row : nullptr, s + 1 < nstrips ? row : nullptr,
-                                         nullptr, ring, ssring, ns, &vend);
+        float vend[DP_RM] = {0.f, 0.f, 0.f, 0.f};
+        int g0 = 0, groups = 0;
+        for (; g0 < ngroups; g0 += groups) {
+            groups = min(DP_RM, ngroups - g0);
+            dp_strip<SC_TM, GAP0, false>(Q, R, prm, P, g0, groups, g0 + groups < ngroups, nullptr, lds, io, vend,
+                                         nullptr);
             __threadfence_block();
         }
-        const float sc = readlane_f(vend, lastlane);
+        // row Lq-1: row r of the last strip, which began at group g0 - groups
+        const int r = P.Lq - 1 - ((g0 - groups) << 6), lane = r / groups;
+        const float v = r - lane * groups == 0 ? vend[0] : r - lane * groups == 1 ? vend[1]
+                        : r - lane * groups == 2 ? vend[2] : vend[3];
+        const float sc = readlane_f(v, __builtin_amdgcn_readfirstlane(lane));
         if (threadIdx.x == 0) scores[o] = sc;
     }
 }
 
 // Row handoff between the waves of one workgroup: wave w sweeps strips
-// w, w+W, ...; strip s writes its last row into ring row s mod W of the pair
-// and publishes, in LDS, how many of its columns are stored.  The wave of
-// strip s+1 waits (bounded spin) until the columns it loads next are there.
-// The rows go through HBM with workgroup-scope release/acquire fences
-// around the LDS progress counters.
+// w, w+W, ... of one row group each.  The last row of a strip goes to the next
+// wave through a ring of MWRING values in LDS, that of wave W-1 to wave 0
+// through the pair's row in HBM.  Per wave two progress words
+// (strip << 16 | columns) in LDS: the columns of its strip's row stored, and
+// the columns of the row above that it has taken.  A strip takes its 16 values
+// of a block when they are stored, and stores its own in the ring when the
+// strip below has taken what they replace (and before its first ones, all of
+// the wave's previous row).  Every wait is a bounded spin and ends: the
+// lowest unfinished strip has its input complete, and the ring it fills is
+// emptied by the strips below it, the last of which (wave W-1) fills a whole
+// row and waits for no one.  That row is overwritten W strips later, each
+// column after every strip between has passed it.  LDS operations of a wave
+// execute in order; the fences of the ring order nothing but LDS, so that no
+// wait includes the backtrace stores, and the row in HBM, whose fences do, is
+// handed over 64 columns at a time.
+constexpr int MWRING = 256;
 template <int W>
-struct LdsSync {
-    int* strip;     // [W] strip each wave is on
-    int* done;      // [W] columns of that strip's row stored
-    int* fail;      // set when a wait gave up
-    __device__ __forceinline__ bool wait(int sp, int cols) {
-        const int pw = sp % W;
+struct RowLds {
+    static constexpr bool IN_LDS = true;
+    float (*rings)[MWRING];
+    unsigned* stored;   // [W]
+    unsigned* taken;    // [W]
+    int* fail;          // set when a wait gave up
+    float* row;         // the pair's row in HBM
+    int s, w;           // this wave's strip and index
+    float wide;         // 64 columns of the row
+    __device__ __forceinline__ bool wait(const unsigned* word, unsigned need) {
         for (long long it = 0;; it++) {
-            const int cs = __hip_atomic_load(strip + pw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const int cd = __hip_atomic_load(done + pw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (cs > sp || (cs == sp && cd >= cols)) break;
+            if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= need) return true;
             if (it > (1ll << 24) || __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
                 __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 return false;
             }
-            __builtin_amdgcn_s_sleep(1);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+    __device__ __forceinline__ void set(unsigned* word, int strip, int cols) {
+        if (lane_id() == 0)
+            __hip_atomic_store(word, ((unsigned)strip << 16) | (unsigned)cols, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ float fetch(int, int) { return 0.f; }
+    __device__ __forceinline__ bool take(float& v, int t0, int Lr) {
+        const int above = (w + W - 1) % W, lane = lane_id();
+        if (w == 0) {
+            if ((t0 & 63) == 0) {
+                if (!wait(stored + above, ((unsigned)(s - 1) << 16) | (unsigned)min(t0 + 64, Lr))) return false;
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                wide = row[min(t0 + lane, Lr - 1)];
+            }
+            v = __shfl(wide, (t0 & 48) + (lane & 15), GTA_WAVE);
+            return true;
+        }
+        const int cols = min(t0 + 16, Lr);
+        if (!wait(stored + above, ((unsigned)(s - 1) << 16) | (unsigned)cols)) return false;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        v = rings[above][(t0 + lane) & (MWRING - 1)];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        set(taken + w, s, cols);
         return true;
     }
-    __device__ __forceinline__ void publish(int s, int cols) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        if (lane_id() == 0) __hip_atomic_store(done + (s % W), cols, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __device__ __forceinline__ void begin(int s) {
-        if (lane_id() == 0) {
-            __hip_atomic_store(done + (s % W), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_store(strip + (s % W), s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __device__ __forceinline__ bool put(int c, int cols, int Lr, float v) {
+        if (cols <= 0) return true;
+        const bool mine = lane_id() >= 48 && c >= 0 && c < Lr;
+        if (w == W - 1) {
+            if (mine) row[c] = v;
+            // a multiple of 64 columns was passed in this block, or the end
+            if ((cols & 63) < 16 || cols >= Lr) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                set(stored + w, s, min(cols, Lr));
+            }
+            return true;
         }
+        cols = min(cols, Lr);
+        const unsigned need = cols > MWRING ? ((unsigned)(s + 1) << 16) | (unsigned)(cols - MWRING)
+                              : s >= W      ? ((unsigned)(s - W + 1) << 16) | (unsigned)Lr
+                                            : 0u;
+        if (need && !wait(taken + w + 1, need)) return false;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        if (mine) rings[w][c & (MWRING - 1)] = v;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        set(stored + w, s, cols);
+        return true;
     }
 };
 
-// DP of one large pair per workgroup of W waves (pairs from plist; ring rows
-// of W x Lr floats per pair at ringoff[item]).  Same cells, codes and walk as
-// k_dp; only the strips run concurrently, pipelined down the query.
+// DP of one pair per workgroup of W waves (pairs from plist).  Same cells and
+// walk as k_dp; only the strips run concurrently, 80 steps apart, down the
+// query.
 template <int SC, bool GAP0, int W>
 __global__ __launch_bounds__(W * GTA_WAVE) void k_dp_mw(DevChunk Q, DevChunk R, DevState S, DpParams prm,
-                                                         const int* plist, float* ring,
-                                                         const unsigned long long* ringoff, int* failflag) {
-    constexpr bool USESS = SC == SC_TMSS;
-    __shared__ int strip[W], done[W], fail;
-    __shared__ float4 cring[W][DPRING];
-    __shared__ float ssring[USESS ? W : 1][USESS ? DPRING : 1];
+                                                         const int* plist, int* failflag) {
+    __shared__ unsigned stored[W], taken[W];
+    __shared__ int fail;
+    __shared__ float rings[W][MWRING];
+    __shared__ DpLds lds[W];
     __shared__ float gtab[SC == SC_SSRR ? NGT * NGT : 1];
     if (SC == SC_SSRR) load_gtab(gtab, prm.rrw);
     DpPair P;
     if (!dp_setup(Q, R, S, prm, plist[blockIdx.x], P)) return;
-    const int w = threadIdx.x / GTA_WAVE;
-    if (threadIdx.x < W) { strip[threadIdx.x] = -1; done[threadIdx.x] = 0; }
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / GTA_WAVE);
+    if (threadIdx.x < W) { stored[threadIdx.x] = 0; taken[threadIdx.x] = 0; }
     if (threadIdx.x == 0) fail = 0;
     __syncthreads();
-    float* rows = ring + ringoff[blockIdx.x];
     unsigned* bt = S.btck + S.btckoff[P.p];
-    const int nstrips = (P.Lq + 63) >> 6;
-    LdsSync<W> sy{strip, done, &fail};
-    for (int s = w; s < nstrips; s += W) {
-        sy.begin(s);
-        const float* rin = s > 0 ? rows + (size_t)((s - 1) % W) * P.Lr : nullptr;
-        float* rout = s + 1 < nstrips ? rows + (size_t)(s % W) * P.Lr : nullptr;
-        if (!dp_strip<SC, GAP0>(Q, R, S, prm, P, s, rin, rout, bt, cring[w], ssring[USESS ? w : 0], sy, nullptr,
-                                gtab))
-            break;
-        // the strip's row is complete
-        sy.publish(s, P.Lr);
+    const int ngroups = (P.Lq + 63) >> 6, nblk = (P.Lr + 63 + 15) >> 4;
+    RowLds<W> io{rings, stored, taken, &fail, S.rowbuf + (size_t)P.qi * (size_t)R.nposs + (size_t)P.rd, 0, w, 0.f};
+    for (int s = w; s < ngroups; s += W) {
+        io.s = s;
+        unsigned* sbt = bt + ((size_t)(s * nblk) << 6);
+        const bool ok = s + 1 < ngroups
+                            ? dp_sweep<SC, GAP0, true, 1, true>(Q, R, prm, P, s, sbt, lds[w], io, nullptr, gtab)
+                            : dp_sweep<SC, GAP0, true, 1, false>(Q, R, prm, P, s, sbt, lds[w], io, nullptr, gtab);
+        if (!ok) break;
     }
     __syncthreads();
     if (fail) {
@@ -1315,58 +1419,60 @@ __global__ __launch_bounds__(W * GTA_WAVE) void k_dp_mw(DevChunk Q, DevChunk R, 
         return;
     }
     dp_count(S, P);
-    if (w == 0) dp_walk(Q, R, S, prm, P, bt);
+    if (w == 0) dp_walk(Q, R, S, prm, P, bt, 1);
 }
 
-// Row handoff between workgroups anywhere on the device (k_dp_grid): strip s
-// of a pair publishes in global memory how many columns of its last row are
-// stored; the strip below waits (bounded spin) for the columns it loads next.
-// Agent-scope release/acquire fences order the row stores and loads.
-struct GridSync {
-    int* done;      // per strip of the pair: columns of its row stored
+// Row handoff between workgroups anywhere on the device (k_dp_grid): every
+// strip has its own row in HBM, filled with ROW_EMPTY (a NaN, which no cell
+// value is) before the launch, and a value itself says that it is there.  The
+// values are relaxed agent-scope atomics of 32 bits, so no fence, cache
+// write-back or counter stands between the store and the load; a strip loads
+// its 16 values a block ahead and again (bounded spin) until all are there.
+constexpr unsigned ROW_EMPTY = 0x7fc0e3d7u;
+struct RowGrid {
+    static constexpr bool IN_LDS = false;
+    const float* in;
+    float* out;
     int* fail;      // set when a wait gave up; every other wait then gives up too
-    __device__ __forceinline__ bool wait(int sp, int cols) {
-        for (long long it = 0;; it++) {
-            const int cd = __hip_atomic_load(done + sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (cd >= cols) break;
+    __device__ __forceinline__ float fetch(int c, int Lr) {
+        return (lane_id() < 16 && c < Lr) ? __hip_atomic_load(in + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                          : 0.f;
+    }
+    __device__ __forceinline__ bool take(float& v, int t0, int Lr) {
+        for (long long it = 0; __any(__float_as_uint(v) == ROW_EMPTY); it++) {
             if (it > (1ll << 22) || __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                 if (lane_id() == 0) __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return false;
             }
-            __builtin_amdgcn_s_sleep(2);
+            v = fetch(t0 + lane_id(), Lr);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         return true;
     }
-    __device__ __forceinline__ void publish(int s, int cols) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        if (lane_id() == 0) __hip_atomic_store(done + s, cols, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __device__ __forceinline__ bool put(int c, int, int Lr, float v) {
+        if (lane_id() >= 48 && c >= 0 && c < Lr)
+            __hip_atomic_store(out + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
     }
 };
 
 // DP fill of a few very large pairs by the whole device: one-wave workgroups
-// take (pair, strip) items in increasing order from a global counter
-// (sync[total]) and sweep them; strip s waits on strip s-1's published row
-// (rows: nstrips x Lr floats per pair at rowoff[k]; strip0[k] is pair k's
-// first item).  Items are handed out in order and a strip waits only on the
-// strip before it, which a running workgroup already holds, so the lowest
-// unfinished strip never waits and the fill always drains.  Same cells and
-// codes as k_dp; k_dp_grid_walk then walks each pair.
+// take (pair, strip) items in increasing order from a global counter and sweep
+// them (strips of one row group; rows: ngroups x Lr floats per pair at
+// rowoff[k]; strip0[k] is pair k's first item).  Items are handed out in order
+// and a strip waits only on the strip before it, which a running workgroup
+// already holds, so the lowest unfinished strip never waits and the fill
+// always drains.  Same cells as k_dp; k_dp_grid_walk then walks each pair.
 template <int SC, bool GAP0>
 __global__ __launch_bounds__(GTA_WAVE) void k_dp_grid(DevChunk Q, DevChunk R, DevState S, DpParams prm,
                                                        const int* plist, int npairs, const int* strip0,
-                                                       int* sync, float* rows, const unsigned long long* rowoff,
+                                                       int* next, float* rows, const unsigned long long* rowoff,
                                                        int* failflag) {
-    __shared__ float4 cring[DPRING];
-    __shared__ float ssring[SC == SC_TMSS ? DPRING : 1];
-    __shared__ float gtab[SC == SC_SSRR ? NGT * NGT : 1];
-    if (SC == SC_SSRR) load_gtab(gtab, prm.rrw);
+    __shared__ DpLds lds;
     const int total = strip0[npairs];
-    int* next = sync + total;
     for (;;) {
         int item = 0;
         if (lane_id() == 0) item = atomicAdd(next, 1);
-        item = __shfl(item, 0, GTA_WAVE);
+        item = __builtin_amdgcn_readfirstlane(__shfl(item, 0, GTA_WAVE));
         if (item >= total) break;
         int lo = 0, hi = npairs - 1;
         while (lo < hi) {
@@ -1376,14 +1482,14 @@ __global__ __launch_bounds__(GTA_WAVE) void k_dp_grid(DevChunk Q, DevChunk R, De
         const int k = lo, s = item - strip0[k];
         DpPair P;
         if (!dp_setup(Q, R, S, prm, plist[k], P)) continue;
-        const int nstrips = strip0[k + 1] - strip0[k];
+        const int ngroups = strip0[k + 1] - strip0[k], nblk = (P.Lr + 63 + 15) >> 4;
         float* prow = rows + rowoff[k];
-        unsigned* bt = S.btck + S.btckoff[P.p];
-        GridSync sy{sync + strip0[k], failflag};
-        const float* rin = s > 0 ? prow + (size_t)(s - 1) * P.Lr : nullptr;
-        float* rout = s + 1 < nstrips ? prow + (size_t)s * P.Lr : nullptr;
-        if (!dp_strip<SC, GAP0>(Q, R, S, prm, P, s, rin, rout, bt, cring, ssring, sy, nullptr, gtab)) break;
-        sy.publish(s, P.Lr);
+        unsigned* bt = S.btck + S.btckoff[P.p] + ((size_t)(s * nblk) << 6);
+        RowGrid io{s > 0 ? prow + (size_t)(s - 1) * P.Lr : nullptr, prow + (size_t)s * P.Lr, failflag};
+        const bool ok = s + 1 < ngroups
+                            ? dp_sweep<SC, GAP0, true, 1, true>(Q, R, prm, P, s, bt, lds, io, nullptr, nullptr)
+                            : dp_sweep<SC, GAP0, true, 1, false>(Q, R, prm, P, s, bt, lds, io, nullptr, nullptr);
+        if (!ok) break;
     }
 }
 
@@ -1397,7 +1503,7 @@ __global__ __launch_bounds__(GTA_WAVE) void k_dp_grid_walk(DevChunk Q, DevChunk 
         return;
     }
     dp_count(S, P);
-    dp_walk(Q, R, S, prm, P, S.btck + S.btckoff[P.p]);
+    dp_walk(Q, R, S, prm, P, S.btck + S.btckoff[P.p], 1);
 }
 
 // ============================================================================
@@ -2373,7 +2479,7 @@ hipError_t launch_dp(const DevChunk& Q, const DevChunk& R, const DevState& S, co
     }
 #define GTA_MW(US, G0, WW, G)                                                                                \
     hipLaunchKernelGGL((k_dp_mw<US, G0, WW>), dim3(B.nmw[G]), dim3(WW * GTA_WAVE), 0, st, Q, R, S, prm, B.mw[G], \
-                       B.ring, B.mwoff[G], B.failflag)
+                       B.failflag)
 #define GTA_KMW4(US, G0) GTA_MW(US, G0, 4, 0)
 #define GTA_KMW8(US, G0) GTA_MW(US, G0, 8, 1)
 #define GTA_KMW16(US, G0) GTA_MW(US, G0, 16, 2)
@@ -2387,18 +2493,22 @@ hipError_t launch_dp(const DevChunk& Q, const DevChunk& R, const DevState& S, co
     if (B.ngrid > 0 && L.usess == SC_SSRR) {
         // The SS/residue fill does not use the device-wide pipeline: its
         // grid-form run stalled on the GPU with no cause found yet.  Those
-        // pairs run as 4-wave workgroups instead, on their grid rows (a pair
-        // holds nstrips >= min(4, nstrips) rows of Lr floats there).
+        // pairs run as 4-wave workgroups instead.
         hipLaunchKernelGGL((k_dp_mw<SC_SSRR, false, 4>), dim3(B.ngrid), dim3(4 * GTA_WAVE), 0, st, Q, R, S, prm,
-                           B.grid, B.ring, B.growoff, B.failflag);
+                           B.grid, B.failflag);
     } else if (B.ngrid > 0) {
-        // progress counters and the item counter start at zero for every fill
-        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((long long)B.gtotal + 1, 256)), dim3(256), 0, st, B.gsync, 0,
-                           (size_t)B.gtotal + 1);
+        // every row empty and the item counter at zero for every fill
+        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((long long)B.growtot, 256)), dim3(256), 0, st, (int*)B.grows,
+                           (int)ROW_EMPTY, B.growtot);
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, B.gnext, 0, (size_t)1);
 #define GTA_KG(US, G0)                                                                                    \
     hipLaunchKernelGGL((k_dp_grid<US, G0>), dim3(B.gworkers), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.grid, \
-                       B.ngrid, B.gstrip0, B.gsync, B.ring, B.growoff, B.failflag)
-        GTA_DPV(GTA_KG);
+                       B.ngrid, B.gstrip0, B.gnext, B.grows, B.growoff, B.failflag)
+        if (L.usess == SC_TMSS) {
+            if (L.gap0) GTA_KG(SC_TMSS, true); else GTA_KG(SC_TMSS, false);
+        } else {
+            if (L.gap0) GTA_KG(SC_TM, true); else GTA_KG(SC_TM, false);
+        }
 #undef GTA_KG
         hipLaunchKernelGGL(k_dp_grid_walk, dim3(B.ngrid), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.grid, B.failflag);
     }

@@ -20,26 +20,22 @@ struct DpLaunch {
     float rrw;         // residue-score weight of kind 2
 };
 
-// Pairs of a chunk split by DP size: the one-wave kernel takes `small`
-// (nullptr: every pair), the W-wave kernel takes `big` with W x Lr floats
-// of ring rows per pair at ringoff[i].
+// Pairs of a chunk split by the form of their DP fill.
 struct DpBuckets {
     const int* small;                       // one wave per pair (nullptr: every pair)
     int nsmall;
-    // one workgroup of W = 4 << g waves per pair, g = 0, 1, 2; ring rows of
-    // W x Lr floats per pair at mwoff[g][k] in ring
+    // one workgroup of W = 4 << g waves per pair, g = 0, 1, 2
     const int* mw[3];
     int nmw[3];
-    const unsigned long long* mwoff[3];
-    float* ring;
     int* failflag;     // set by a W-wave or grid fill whose row wait gave up
     // pairs filled by the device-wide strip pipeline (k_dp_grid)
     const int* grid;
     int ngrid;
     const int* gstrip0;                     // [ngrid + 1] first strip item of each pair
-    int gtotal;                             // strips of all grid pairs
-    int* gsync;                             // [gtotal + 1] strip progress, then the item counter
-    const unsigned long long* growoff;      // per pair nstrips x Lr floats at growoff[k] in ring
+    int* gnext;                             // the item counter
+    float* grows;                           // per pair nstrips x Lr floats at growoff[k]
+    const unsigned long long* growoff;
+    size_t growtot;                         // floats of all grid pairs' rows
     int gworkers;                           // one-wave workgroups of the fill
     // any pair outside the one-wave list
     bool any_big() const { return nmw[0] > 0 || nmw[1] > 0 || nmw[2] > 0 || ngrid > 0; }
