@@ -116,11 +116,12 @@ struct gta_ctx {
     // counter of the device-wide fill
     DevBuf s_dpbig, s_grows, s_growoff, s_fail, s_gstrip0, s_gnext;
     DpBuckets dpb{};
-    // a pair is filled by several waves when Lq*Lr >= mw_min_cells and it
-    // has at least mw_min_strips 64-row strips (and Lr >= 256)
+    // a pair is large when Lq*Lr >= mw_min_cells and it has at least
+    // mw_min_strips groups of 64 rows (and Lr >= 256)
     long long mw_min_cells = 1ll << 22;
     int mw_min_strips = 16;
-    // those pairs are pipelined over the whole device instead when they number
+    bool dp_forced = false;     // thresholds set by gta_test_set_dp_buckets
+    // those pairs are pipelined over the whole device when they number
     // at most half the CUs (dp_grid 0), always (1) or never (2)
     int dp_grid = 0;
     // per pair: DP launch form (DPF_*) of the resident chunks
@@ -394,12 +395,14 @@ static Geom make_geom(const gta_ctx* c) {
 // Every pair's fill runs in one of five forms: one wave (k_dp), one workgroup
 // of 4, 8 or 16 waves (k_dp_mw) or the device-wide strip pipeline
 // (k_dp_grid).  By default large pairs (Lq*Lr >= mw_min_cells, >= mw_min_strips
-// strips, Lr >= 256) take the grid form when they number at most half the CUs
-// and the W-wave form otherwise.  With autotuning on, pairs of >= 4 strips and
-// >= 2^18 cells are grouped by length bucket (log2 of strips, log2 of Lr,
-// log2 of the bucket's pair count) and each bucket's form is the fastest of
-// the candidates in a timed fill of the whole chunk, kept per context and in
-// the cache file.
+// groups of 64 rows, Lr >= 256) that number at most half the CUs take the grid
+// form, and the others one wave or, in a small chunk, one workgroup
+// (default_dp_forms); gta_test_set_dp_buckets puts the large ones into a
+// workgroup and the others into one wave instead.  With autotuning on, pairs
+// of >= 4 groups and >= 2^18 cells are grouped by length bucket (log2 of the
+// groups, log2 of Lr, log2 of the bucket's pair count) and each bucket's form
+// is the fastest of the candidates in a timed fill of the whole chunk, kept per
+// context and in the cache file.
 enum { DPF_ONE = 0, DPF_W4 = 1, DPF_W8 = 2, DPF_W16 = 3, DPF_GRID = 4, DPF_N = 5 };
 
 static int ilog2ll(long long v) {
@@ -464,24 +467,56 @@ static int upload_dp_buckets(gta_ctx* c, const std::vector<unsigned char>& form,
     return GTA_OK;
 }
 
+// A chunk of at most two pairs per CU leaves most of the device idle, and its
+// launches last as long as the longest fill.  One wave takes 0.05 us per step
+// and row of a lane (measured: 65 us for 256 x 256, 0.23 ms for 500 x 500, 0.85
+// ms for 1,000 x 1,000 residues), one workgroup of W waves 0.08 us per step with
+// the strips 80 steps apart (45 us, 0.11 ms and, with 16 waves, 0.2 ms for the
+// same pairs): there, a pair that a workgroup fills in 3/4 of the time or less
+// takes the smallest workgroup that holds its strips.  In larger chunks one
+// wave per pair is faster on the whole (40,000 pairs of 256 x 256: 2.2 against
+// 4.0 ms, 1,600: 0.17 against 0.21 ms; the longest tenth in workgroups cost the
+// 30 fills of a 4 x 1,500 search 5 of 11 ms, as their launch follows the
+// other's).
+constexpr double DP_US_ROWSTEP = 0.05, DP_US_MWSTEP = 0.08;
+
+static int dp_mw_form(int strips) { return strips <= 4 ? DPF_W4 : strips <= 8 ? DPF_W8 : DPF_W16; }
+
 static void default_dp_forms(const gta_ctx* c, std::vector<unsigned char>& form) {
     const int nq = c->q.nstrs, nr = c->r.nstrs;
     std::vector<int> big;
     int minstrips = 1 << 30;
     for (int qi = 0; qi < nq; qi++) {
         const int Lq = c->q.len[qi], ns = (Lq + 63) / 64;
+        if (ns < c->mw_min_strips) continue;
         for (int ri = 0; ri < nr; ri++) {
             const int Lr = c->r.len[ri];
-            if ((long long)Lq * Lr >= c->mw_min_cells && ns >= c->mw_min_strips && Lr >= 256) {
+            if ((long long)Lq * Lr >= c->mw_min_cells && Lr >= 256) {
                 big.push_back(qi * nr + ri);
                 minstrips = std::min(minstrips, ns);
             }
         }
     }
-    if (big.empty()) return;
-    const bool grid = c->dp_grid == 1 || (c->dp_grid == 0 && (int)big.size() * 2 <= c->ncu);
-    const int f = grid ? DPF_GRID : (minstrips >= 32 ? DPF_W16 : (minstrips >= 16 ? DPF_W8 : DPF_W4));
-    for (int pidx : big) form[pidx] = (unsigned char)f;
+    const bool grid = !big.empty() && (c->dp_grid == 1 || (c->dp_grid == 0 && (int)big.size() * 2 <= c->ncu));
+    // large pairs that are too many for the grid form fill the device's wave
+    // slots (16 a CU) with workgroups until they do so with one wave each
+    if (!big.empty() && !grid && (c->dp_forced || (long long)big.size() <= 16ll * c->ncu)) {
+        const int f = minstrips >= 32 ? DPF_W16 : (minstrips >= 16 ? DPF_W8 : DPF_W4);
+        for (int pidx : big) form[pidx] = (unsigned char)f;
+    }
+    if (grid)
+        for (int pidx : big) form[pidx] = DPF_GRID;
+    if (c->dp_forced) return;
+    if ((long long)nq * nr > 2ll * c->ncu) return;
+    for (int qi = 0; qi < nq; qi++) {
+        const int G = (c->q.len[qi] + 63) / 64, f = dp_mw_form(G), W = 4 << (f - DPF_W4);
+        for (int ri = 0; ri < nr; ri++) {
+            unsigned char& fm = form[(size_t)qi * nr + ri];
+            const double steps = c->r.len[ri] + 63.0;
+            const double mw = DP_US_MWSTEP * ((G + W - 1) / W) * (steps + 80.0 * (std::min(W, G) - 1));
+            if (fm == DPF_ONE && mw <= 0.75 * DP_US_ROWSTEP * G * steps) fm = (unsigned char)f;
+        }
+    }
 }
 
 // time of one DP fill of the whole chunk under the given forms (ms)
@@ -1051,6 +1086,7 @@ int gta_test_set_dp_buckets(gta_ctx* c, long long min_cells, int min_strips) {
     if (!c || min_cells < 0 || min_strips < 1) return fail(c, GTA_ERR_ARG, "invalid DP bucket thresholds");
     c->mw_min_cells = min_cells;
     c->mw_min_strips = min_strips;
+    c->dp_forced = true;
     c->gvalid = false;   // the captured graph holds the old launch forms and buffers
     return GTA_OK;
 }

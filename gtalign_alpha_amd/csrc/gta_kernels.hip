@@ -753,8 +753,11 @@ __device__ __forceinline__ void load_gtab(float* gtab, float rrw) {
 // each, the last one the groups that are left.  One wave per pair takes
 // rm = 4: the ring read, the cross-lane shift, the block bookkeeping and the 63
 // skewed steps are paid once per four rows, and four independent cell scores
-// are in flight.  The forms that run a pair's strips in parallel take rm = 1.
-constexpr int DP_RM = 4;
+// are in flight.  The forms that run a pair's strips in parallel, which are
+// there for a short launch, take rm = 1: a step then takes 80 ns against 130
+// with rm = 2 (one pair of 500 x 500: 90 against 104 us, 400 x 3,000: 290
+// against 430 us).
+constexpr int DP_RM = 4, MW_RM = 1;
 // Waves per SIMD that the one-wave kernel is compiled for: 128 registers hold
 // an unrolled block of 8 steps of four rows without spills in it.  DP of a
 // 16 x 12,000 search, 30 fills: 3 waves 110.2 ms, 4 105.6, 5 110.9, 6 120.0,
@@ -1093,6 +1096,12 @@ __device__ __forceinline__ bool dp_strip(const DevChunk& Q, const DevChunk& R, c
     }
 }
 
+// the 2-bit code of field f (0-63) of four words
+__device__ __forceinline__ unsigned field4(unsigned c0, unsigned c1, unsigned c2, unsigned c3, int f) {
+    const unsigned lo = (f & 16) ? c1 : c0, hi = (f & 16) ? c3 : c2;
+    return (((f & 32) ? hi : lo) >> ((f & 15) << 1)) & 3u;
+}
+
 // Backtrace walk from the bottom-right cell (BtckToMatched, btck2match.cuh:46-52;
 // ConstrainedBtckToMatched keeps pairs within d8 and their d2).  Matched pairs
 // are stored in walk (reverse) order.
@@ -1101,10 +1110,12 @@ __device__ __forceinline__ bool dp_strip(const DevChunk& Q, const DevChunk& R, c
 // y0 - l in the 64 columns around the diagonal through the window's first
 // cell (x0 - l - 31 to x0 - l + 32, field f), loaded at once (5 words a lane).
 // A diagonal move keeps f, a move left lowers it, a move up raises it, so a run
-// of diagonal moves is one ballot over the window and every other move one
-// lane's code; no memory access stands between two moves.  A window ends
-// with its rows or when the path leaves its columns.  With one memory access
-// per change of direction the walk took about as long as the fill.
+// of moves in one direction is found by one ballot over the window's rows
+// (diagonal, up) or over the fields of one row (left), and no memory access
+// stands between two runs.  A window ends with its rows or when the path leaves
+// its columns; its matched pairs are stored while the next window's codes are
+// on their way.  Bound by latency: with one memory access per run the walk
+// took about as long as the fill; a 250-residue walk now takes 5-6 windows.
 __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S, const DpParams& prm,
                         const DpPair& P, const unsigned* bt, int rm) {
     const int lane = lane_id();
@@ -1127,61 +1138,85 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
     const bool constrained = prm.mode == DPM_CONSTRAINED;
     const float d82 = GetD82(Lq, Lr);
     int y0 = Lq - 1, x0 = Lr - 1, k = 0;
-    while (y0 >= 0 && x0 >= 0) {
+    int ym = 0, xm = -1;        // the lane's matched row and column of the last window
+    for (;;) {
+        const bool more = y0 >= 0 && x0 >= 0;
         const int yy = y0 - lane;
-        unsigned c0, c1, c2, c3;    // the codes of fields 0-15, 16-31, 32-47, 48-63
-        {
+        unsigned v[5] = {0, 0, 0, 0, 0}, sh = 0;
+        if (more) {
             int rows, ln;
             const unsigned* w = code_row(bt, nblk, rm, ngroups, max(yy, 0), rows, ln);
             const int t = x0 - lane - 31 + ln, tb = t >> 4;     // step of field 0
-            unsigned v[5];
 #pragma unroll
             for (int i = 0; i < 5; i++) v[i] = w[(size_t)(min(max(tb + i, 0), nblk - 1) * rows) << 6];
-            const unsigned sh = (unsigned)(t & 15) << 1;
-            c0 = __builtin_amdgcn_alignbit(v[1], v[0], sh);
-            c1 = __builtin_amdgcn_alignbit(v[2], v[1], sh);
-            c2 = __builtin_amdgcn_alignbit(v[3], v[2], sh);
-            c3 = __builtin_amdgcn_alignbit(v[4], v[3], sh);
+            sh = (unsigned)(t & 15) << 1;
         }
-        int l = 0, f = 31, xm = -1;     // xm: the lane's matched column
-        for (;;) {
-            const unsigned c = f < 32 ? (f < 16 ? c0 : c1) : (f < 48 ? c2 : c3);
-            // cells left of or above the matrix end the walk
-            const int col = x0 - lane - 31 + f;
-            const unsigned code = (yy >= 0 && col >= 0) ? (c >> ((f & 15) << 1)) & 3u : (unsigned)BT_STOP;
+        // the last window's matched pairs
+        bool keep = xm >= 0;
+        if (__any(keep)) {
+            float qx = 0, qy = 0, qz = 0, rx = 0, ry = 0, rz = 0, d2 = 0;
+            if (keep) {
+                qx = Q.x[qd + ym]; qy = Q.y[qd + ym]; qz = Q.z[qd + ym];
+                rx = R.x[rd + xm]; ry = R.y[rd + xm]; rz = R.z[rd + xm];
+                if (constrained) {
+                    d2 = tfm_dist2(P.tfm, qx, qy, qz, rx, ry, rz);
+                    keep = d2 <= d82;
+                }
+            }
+            const unsigned long long km = __ballot(keep);
+            if (keep) {
+                const int o = k + __popcll(km & ((1ull << lane) - 1ull));
+                aqx[o] = qx; aqy[o] = qy; aqz[o] = qz;
+                arx[o] = rx; ary[o] = ry; arz[o] = rz;
+                aqp[o] = (float)ym; arp[o] = (float)xm;
+                if (constrained) ad2[o] = d2;
+            }
+            k += __popcll(km);
+        }
+        if (!more) break;
+        // the codes of fields 0-15, 16-31, 32-47, 48-63
+        const unsigned c0 = __builtin_amdgcn_alignbit(v[1], v[0], sh), c1 = __builtin_amdgcn_alignbit(v[2], v[1], sh),
+                       c2 = __builtin_amdgcn_alignbit(v[3], v[2], sh), c3 = __builtin_amdgcn_alignbit(v[4], v[3], sh);
+        int l = 0, f = 31, singles = 0;     // singles: moves left or up since the last diagonal run
+        ym = yy;
+        xm = -1;
+        const int col0 = x0 - lane - 31;    // the lane's column of field 0
+        do {
+            // cells left of or above the matrix stop the walk
+            const unsigned code = (yy >= 0 && col0 + f >= 0) ? field4(c0, c1, c2, c3, f) : (unsigned)BT_STOP;
             const unsigned long long diag = __ballot(code == BT_DIAG) >> l;
             if (diag & 1ull) {
                 const int run = ~diag ? (int)__builtin_ctzll(~diag) : GTA_WAVE;     // at most 64 - l
-                if (lane >= l && lane < l + run) xm = col;
+                if (lane >= l && lane < l + run) xm = col0 + f;
                 l += run;
+                singles = 0;
+                continue;
+            }
+            const unsigned here = __builtin_amdgcn_readlane(code, l);
+            if (here == BT_STOP) {
+                l = GTA_WAVE;
+                y0 = -1;        // the walk has left the matrix
+            } else if (++singles < 4) {
+                // most gaps are short: one move at a time is cheaper than a run's ballot
+                if (here == BT_UP) { l++; f++; } else f--;
+            } else if (here == BT_UP) {
+                // rows l, l+1, ... at fields f, f+1, ...
+                const int fl = f + lane - l;
+                const unsigned long long up = __ballot(fl < GTA_WAVE && yy >= 0 && col0 + fl >= 0 &&
+                                                       field4(c0, c1, c2, c3, fl) == BT_UP) >> l;
+                const int run = ~up ? (int)__builtin_ctzll(~up) : GTA_WAVE;
+                l += run;
+                f += run;
             } else {
-                const unsigned here = __builtin_amdgcn_readlane(code, l);
-                if (here == BT_UP) { l++; f++; }
-                else if (here == BT_LEFT) f--;
-                else { l = -1; break; }
+                // row l at fields f, f-1, ...: lane i looks at field f - i
+                const unsigned r0 = __builtin_amdgcn_readlane(c0, l), r1 = __builtin_amdgcn_readlane(c1, l),
+                               r2 = __builtin_amdgcn_readlane(c2, l), r3 = __builtin_amdgcn_readlane(c3, l);
+                const bool left = lane <= f && x0 - l - 31 + f - lane >= 0 &&
+                                  field4(r0, r1, r2, r3, max(f - lane, 0)) == BT_LEFT;
+                const unsigned long long lm = __ballot(left);
+                f -= ~lm ? (int)__builtin_ctzll(~lm) : GTA_WAVE;
             }
-            if (l >= GTA_WAVE || f < 0 || f > 63) break;
-        }
-        float qx = 0, qy = 0, qz = 0, rx = 0, ry = 0, rz = 0, d2 = 0;
-        bool keep = xm >= 0;
-        if (keep) {
-            qx = Q.x[qd + yy]; qy = Q.y[qd + yy]; qz = Q.z[qd + yy];
-            rx = R.x[rd + xm]; ry = R.y[rd + xm]; rz = R.z[rd + xm];
-            if (constrained) {
-                d2 = tfm_dist2(P.tfm, qx, qy, qz, rx, ry, rz);
-                keep = d2 <= d82;
-            }
-        }
-        const unsigned long long km = __ballot(keep);
-        if (keep) {
-            const int o = k + __popcll(km & ((1ull << lane) - 1ull));
-            aqx[o] = qx; aqy[o] = qy; aqz[o] = qz;
-            arx[o] = rx; ary[o] = ry; arz[o] = rz;
-            aqp[o] = (float)yy; arp[o] = (float)xm;
-            if (constrained) ad2[o] = d2;
-        }
-        k += __popcll(km);
-        if (l < 0) break;
+        } while (l < GTA_WAVE && f >= 0 && f < GTA_WAVE);
         y0 -= l;
         x0 += f - 31 - l;
     }
@@ -1299,7 +1334,7 @@ __global__ __launch_bounds__(GTA_WAVE) void k_dp_score(DevChunk Q, DevChunk R, D
 }
 
 // Row handoff between the waves of one workgroup: wave w sweeps strips
-// w, w+W, ... of one row group each.  The last row of a strip goes to the next
+// w, w+W, ... of MW_RM row groups.  The last row of a strip goes to the next
 // wave through a ring of MWRING values in LDS, that of wave W-1 to wave 0
 // through the pair's row in HBM.  Per wave two progress words
 // (strip << 16 | columns) in LDS: the columns of its strip's row stored, and
@@ -1405,12 +1440,13 @@ __global__ __launch_bounds__(W * GTA_WAVE) void k_dp_mw(DevChunk Q, DevChunk R, 
     unsigned* bt = S.btck + S.btckoff[P.p];
     const int ngroups = (P.Lq + 63) >> 6, nblk = (P.Lr + 63 + 15) >> 4;
     RowLds<W> io{rings, stored, taken, &fail, S.rowbuf + (size_t)P.qi * (size_t)R.nposs + (size_t)P.rd, 0, w, 0.f};
-    for (int s = w; s < ngroups; s += W) {
+    for (int s = w; s * MW_RM < ngroups; s += W) {
         io.s = s;
-        unsigned* sbt = bt + ((size_t)(s * nblk) << 6);
-        const bool ok = s + 1 < ngroups
-                            ? dp_sweep<SC, GAP0, true, 1, true>(Q, R, prm, P, s, sbt, lds[w], io, nullptr, gtab)
-                            : dp_sweep<SC, GAP0, true, 1, false>(Q, R, prm, P, s, sbt, lds[w], io, nullptr, gtab);
+        const int g0 = s * MW_RM, groups = min(MW_RM, ngroups - g0);
+        unsigned* sbt = bt + ((size_t)(g0 * nblk) << 6);
+        const bool ok = g0 + groups < ngroups
+                            ? dp_sweep<SC, GAP0, true, MW_RM, true>(Q, R, prm, P, g0, sbt, lds[w], io, nullptr, gtab)
+                            : dp_sweep<SC, GAP0, true, MW_RM, false>(Q, R, prm, P, g0, sbt, lds[w], io, nullptr, gtab);
         if (!ok) break;
     }
     __syncthreads();
@@ -1419,7 +1455,7 @@ __global__ __launch_bounds__(W * GTA_WAVE) void k_dp_mw(DevChunk Q, DevChunk R, 
         return;
     }
     dp_count(S, P);
-    if (w == 0) dp_walk(Q, R, S, prm, P, bt, 1);
+    if (w == 0) dp_walk(Q, R, S, prm, P, bt, MW_RM);
 }
 
 // Row handoff between workgroups anywhere on the device (k_dp_grid): every

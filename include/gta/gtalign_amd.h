@@ -223,7 +223,7 @@ int gta_dp_cell_counts(const gta_ctx* ctx, double* useful, double* launched);
  * Each pair's DP fill runs as one wave, as one workgroup of 4, 8 or 16 waves,
  * or pipelined over the whole device.  Off (the default), large pairs take
  * the grid form when they number at most half the compute units and the
- * W-wave form otherwise.  On, pairs of >= 4 strips of 64 rows and >= 2^18
+ * W-wave form otherwise, and small chunks the W-wave form.  On, pairs of >= 4 strips of 64 rows and >= 2^18
  * cells are grouped by length bucket (log2 of the strip count, log2 of the
  * reference length, log2 of the bucket's pair count); at the first
  * gta_process on a chunk pair, each bucket without a cached choice is timed

@@ -41,10 +41,11 @@ int gta_test_dp_score(gta_ctx* ctx, const float* tfms, const int* slotflags, int
 
 /* Thresholds of the DP's size buckets: a pair is filled by a workgroup of
  * several waves (strips pipelined down the query) when Lq*Lr >= min_cells,
- * it has at least min_strips 64-row strips and Lr >= 256; otherwise by one
- * wave.  Defaults 4,194,304 cells and 16 strips.  Takes effect at the next
- * gta_process / gta_test_dp.  Lets tests drive the multi-wave fill on
- * moderate sizes. */
+ * it has at least min_strips groups of 64 rows and Lr >= 256; otherwise by
+ * one wave.  Before the first call: 4,194,304 cells and 16 groups, and in
+ * chunks of at most two pairs per CU every pair that several waves fill in 3/4
+ * of the time or less.  Takes effect at the next gta_process / gta_test_dp.
+ * Lets tests drive the multi-wave fill on moderate sizes. */
 int gta_test_set_dp_buckets(gta_ctx* ctx, long long min_cells, int min_strips);
 
 /* Pairs of the multi-wave bucket above are filled by the whole device
