@@ -743,20 +743,28 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
     return GTA_OK;
 }
 
-// Waves per workgroup of the DPRefine launches.  One-wave workgroups leave
-// fewer of a CU's lanes idle while a pair's last slots run, but stage only
-// alignments of up to rlds_cap32(1) positions in LDS; longer ones are read from
-// L2 in every pass.  An alignment is at most min(Lq, Lr) long, so one wave is
-// used when at most 15% of the chunks' pairs can have longer alignments (16 x
-// 50,000 workload: 7%, DPRefine 0.85 -> 0.79 s with one wave; 1 x 500,000: 27%,
-// 0.40 -> 0.50 s).
+// Waves per workgroup of the DPRefine launches.  A launch ends with its longest
+// alignments, whose slots (about 6 per 40 positions) wait for each other in
+// the workgroup's 8 slot groups a wave, so larger workgroups make it shorter
+// until the device is full of them; then smaller ones leave fewer lanes idle
+// while a pair's last slots run.  28 launches with 1, 2 and 4 waves: 1 x 256
+// pairs 9.8, 6.4, 4.9 ms; 4 x 1,500 26.8, 16.4, 13.2; 4 x 2,500 85.7, 40.4, 27.1
+// (33 launches); 8 x 1,500 85.7, 41.4, 39.7; 1 x 25,000 64, 44.6, 47.0; 16 x
+// 12,000 202, 205, 258 (8 waves: 5.1, 18.7, 39, 62, 78, 455).  One-wave
+// workgroups also stage only alignments of up to rlds_cap32(1) positions in
+// LDS; longer ones are read from L2 in every pass.  An alignment is at most
+// min(Lq, Lr) long, so one wave is used when at most 15% of the pairs can have
+// longer ones (16 x 50,000: 7%, 0.85 s with two waves, 0.79 with one; 1 x
+// 500,000: 27%, 0.40 and 0.50).
 static int dprefine_waves(const gta_ctx* c) {
+    const double np = (double)c->q.len.size() * (double)c->r.len.size();
+    if (np <= 64.0 * c->ncu) return 4;
+    if (np <= 1024.0 * c->ncu) return 2;
     const int cap = rlds_cap32(1);
     long long ql = 0, rl = 0;
     for (int v : c->q.len) ql += v > cap;
     for (int v : c->r.len) rl += v > cap;
-    const double np = (double)c->q.len.size() * (double)c->r.len.size();
-    return (np > 0 && (double)ql * (double)rl <= 0.15 * np) ? 1 : 2;
+    return (double)ql * (double)rl <= 0.15 * np ? 1 : 2;
 }
 
 static int run_stage(gta_ctx* c, double* seconds, double* cells) {
@@ -806,7 +814,8 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
         HIPCHK(c, ev_end());                 \
     } while (0)
     int maxaln = std::min(c->q.len.front(), c->r.len.front());
-    RefineLaunch RL{dinv, 0, 0, 0, 0.f, std::min(maxaln, 1536), dprefine_waves(c)};
+    const int dpr_waves = dprefine_waves(c);
+    RefineLaunch RL{dinv, 0, 0, 0, 0.f, std::min(maxaln, 1536), 0};
     // After each filter (the stage-1 prescreen, the -s threshold) the live
     // pairs are listed on the device.  The batched form's launches that follow
     // are persistent grids draining those lists (no host round trip: the
@@ -821,7 +830,7 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
     int* listc = c->dpb.any_big() ? c->s_listc.as<int>() : nullptr;
     int* ltot = c->s_ltot.as<int>();
     int* heads = batched ? c->s_heads.as<int>() : nullptr;
-    const int pgrid_dp = c->ncu * 32, pgrid_rf = c->ncu * REFINE_WGS_PER_CU;
+    const int pgrid_dp = c->ncu * 32;
     DpBuckets dpb = c->dpb;         // plain form: one-wave list narrowed to live pairs
     RefSplit rsp = c->rsp;
     auto queue = [&](const int* items, const int* count) -> WorkQ {
@@ -846,8 +855,9 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
     auto refine = [&](int mode, int epi, int dpi, int maxdpi, float prescore) -> hipError_t {
         RefineLaunch L = RL;
         L.epi = epi; L.dpi = dpi; L.maxndpiters = maxdpi; L.prescore = prescore;
+        L.waves = mode == RM_DPREFINE_L ? dpr_waves : FINAL_WAVES;
         // a persistent grid keeps 16 waves per CU whatever the workgroup size
-        const int pg = (mode == RM_DPREFINE_L && L.waves == 1) ? c->ncu * 16 : pgrid_rf;
+        const int pg = c->ncu * 16 / L.waves;
         return launch_refine_dp(prec, mode, Q, R, S, G, L, rsp, queue(listb, ltot + 1), pg, st);
     };
     // DPRefine<GAP0,PRESCREEN> (MpStage1.cpp:455-510)

@@ -2568,10 +2568,9 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
                             const Geom& G, const RefineLaunch& L, const RefSplit& Sp, const WorkQ& wq,
                             int pgrid, hipStream_t st) {
     RefineParams prm{L.dinv, L.epi, L.dpi, L.maxndpiters, L.prescore};
-    // DPRefine runs in workgroups of L.waves (1 or 2), the other modes in 2-wave ones
-    const bool w1 = mode == RM_DPREFINE && L.waves == 1;
-    const int ldscap = (prec == 0 || mode == RM_DPREFINE) ? std::min(L.ldscap, rlds_cap32(w1 ? 1 : RWAVES))
-                                                          : L.ldscap;
+    // waves per workgroup of the unsplit pairs (the log search keeps RWAVES)
+    const int W = mode == RM_PROD2L ? RWAVES : L.waves;
+    const int ldscap = mode == RM_DPREFINE ? std::min(L.ldscap, rlds_cap32(W)) : L.ldscap;
     const size_t lds = (size_t)ldscap * 6 * sizeof(float);
     const int nsmall = wq.items ? pgrid : (Sp.small ? Sp.nsmall : S.nq * S.nr);
     const bool phase2 = (mode == RM_FIN2 || mode == RM_PROD2);
@@ -2581,31 +2580,22 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
                                             Sp.slots_per_part)
                                : 1;
     SlotBest* parts = (SlotBest*)Sp.partbuf;
-#define GTA_RL(PP, MM)                                                                                        \
-    do {                                                                                                      \
-        if (nsmall > 0)                                                                                       \
-            hipLaunchKernelGGL((k_refine_dp<PP, MM>), dim3(nsmall), dim3(RTHREADS), lds, st, Q, R, S, G, prm, \
-                               ldscap, Sp.small, (SlotBest*)nullptr, wq);                                   \
-        if (Sp.nbig > 0) {                                                                                    \
-            hipLaunchKernelGGL((k_refine_dp<PP, MM>), dim3(Sp.nbig, np), dim3(RTHREADS), lds, st, Q, R, S, G, \
-                               prm, ldscap, Sp.big, parts, WorkQ{});                                        \
-            hipLaunchKernelGGL((k_merge_parts<2, MM>), dim3((Sp.nbig + 63) / 64), dim3(64), 0, st, Q, R, S,  \
-                               prm, Sp.big, Sp.nbig, np, parts);                                              \
-        }                                                                                                     \
-    } while (0)
-    // the same with 1-wave workgroups
-#define GTA_RL1(PP, MM)                                                                                        \
+    // pairs of the small bucket (or the queue's) in workgroups of W waves, split
+    // pairs in workgroups of WB
+#define GTA_RLW(PP, MM, W, WB)                                                                                 \
     do {                                                                                                       \
         if (nsmall > 0)                                                                                        \
-            hipLaunchKernelGGL((k_refine_dp<PP, MM, 1>), dim3(nsmall), dim3(GTA_WAVE), lds, st, Q, R, S, G, prm, \
+            hipLaunchKernelGGL((k_refine_dp<PP, MM, W>), dim3(nsmall), dim3(W * GTA_WAVE), lds, st, Q, R, S, G, prm, \
                                ldscap, Sp.small, (SlotBest*)nullptr, wq);                                    \
         if (Sp.nbig > 0) {                                                                                     \
-            hipLaunchKernelGGL((k_refine_dp<PP, MM, 1>), dim3(Sp.nbig, np), dim3(GTA_WAVE), lds, st, Q, R, S, G, \
-                               prm, ldscap, Sp.big, parts, WorkQ{});                                         \
+            hipLaunchKernelGGL((k_refine_dp<PP, MM, WB>), dim3(Sp.nbig, np), dim3(WB * GTA_WAVE), lds, st, Q, R, S, \
+                               G, prm, ldscap, Sp.big, parts, WorkQ{});                                      \
             hipLaunchKernelGGL((k_merge_parts<2, MM>), dim3((Sp.nbig + 63) / 64), dim3(64), 0, st, Q, R, S,   \
                                prm, Sp.big, Sp.nbig, np, parts);                                               \
         }                                                                                                      \
     } while (0)
+    // the final stage's modes
+#define GTA_RL(PP, MM) GTA_RLW(PP, MM, FINAL_WAVES, RWAVES)
     // the log search's steps run in order within one workgroup: no split
 #define GTA_RL_LOG(PP)                                                                                         \
     do {                                                                                                       \
@@ -2619,8 +2609,9 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
 #define GTA_RLM(PP)                                      \
     switch (mode) {                                      \
         case RM_DPREFINE:                                \
-            if (w1) GTA_RL1(0, RM_DPREFINE);             \
-            else GTA_RL(0, RM_DPREFINE);                 \
+            if (W == 1) GTA_RLW(0, RM_DPREFINE, 1, 1);   \
+            else if (W == 2) GTA_RLW(0, RM_DPREFINE, 2, 2); \
+            else GTA_RLW(0, RM_DPREFINE, 4, RWAVES);     \
             break;                                       \
         case RM_FIN1: GTA_RL(PP, RM_FIN1); break;         \
         case RM_FIN2: GTA_RL(PP, RM_FIN2); break;         \
@@ -2633,8 +2624,8 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
     if (prec) { GTA_RLM(1) } else { GTA_RLM(0) }
 #undef GTA_RLM
 #undef GTA_RL_LOG
-#undef GTA_RL1
 #undef GTA_RL
+#undef GTA_RLW
     return hipGetLastError();
 }
 hipError_t launch_prod_aln(const DevChunk& Q, const DevChunk& R, const DevState& S, char* alns, int nodel,
