@@ -17,12 +17,38 @@ namespace gta {
 template <typename T> __device__ __forceinline__ T t_sqrt(T x);
 template <> __device__ __forceinline__ float t_sqrt<float>(float x) { return sqrtf(x); }
 template <> __device__ __forceinline__ double t_sqrt<double>(double x) { return sqrt(x); }
-template <typename T> __device__ __forceinline__ T t_abs(T x) { return x < (T)0 ? -x : x; }
+// |x| as an operand modifier
+__device__ __forceinline__ float t_abs(float x) { return fabsf(x); }
+__device__ __forceinline__ double t_abs(double x) { return fabs(x); }
+// The solve's divisions and square roots, correctly rounded as the plain
+// operators are, without their scaling and special cases (operands here are
+// normal and far from the exponent limits).  Checked on gfx950 against the
+// operators: the square root over every mantissa at both exponent parities, the
+// reciprocal over every mantissa, the division over every pair of mantissas
+// (div_rn_pos, gta_device.h).  In single precision a square root takes 5
+// instructions instead of 15, its reciprocal 8 instead of 26, a further
+// division by the same number 3 instead of 11.
+__device__ __forceinline__ float t_sqrt_pos(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), g = __fmul_rn(x, y);
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), __fmul_rn(0.5f, y), g);
+}
+__device__ __forceinline__ double t_sqrt_pos(double x) { return sqrt(x); }
+__device__ __forceinline__ float t_rcp(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ double t_rcp(double b) { return 1.0 / b; }
+// a / b, y = t_rcp(b)
+__device__ __forceinline__ float t_div(float a, float b, float y) {
+    const float q = __fmul_rn(a, y);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+__device__ __forceinline__ double t_div(double a, double b, double) { return a / b; }
 template <typename T> __device__ __forceinline__ T t_atan2(T y, T x);
 template <> __device__ __forceinline__ float t_atan2<float>(float y, float x) { return atan2f(y, x); }
 template <> __device__ __forceinline__ double t_atan2<double>(double y, double x) { return atan2(y, x); }
 template <typename T> __device__ __forceinline__ void t_sincos(T a, T& s, T& c);
-template <> __device__ __forceinline__ void t_sincos<float>(float a, float& s, float& c) { s = sinf(a); c = cosf(a); }
+template <> __device__ __forceinline__ void t_sincos<float>(float a, float& s, float& c) { sincosf(a, &s, &c); }
 template <> __device__ __forceinline__ void t_sincos<double>(double a, double& s, double& c) { s = sin(a); c = cos(a); }
 
 template <typename T>
@@ -57,9 +83,9 @@ __device__ __forceinline__ bool SolveCubic(T det, T spur, T cof, T& e0, T& e1, T
     T h = spur * spur - cof;
     if (h <= (T)0) return false;
     T g = (spur * cof - det * det) * (T)0.5 - spur * h;
-    T sqrth = t_sqrt(h);
+    T sqrth = t_sqrt_pos(h);
     T hh = h * h * h - g * g;
-    T d = t_atan2(t_sqrt(hh > (T)0 ? hh : (T)0), -g) * ((T)1 / (T)3);
+    T d = t_atan2(hh > (T)0 ? t_sqrt_pos(hh) : (T)0, -g) * ((T)1 / (T)3);
     T sth, cth;
     t_sincos(d, sth, cth);
     cth = sqrth * cth;
@@ -94,7 +120,7 @@ __device__ __forceinline__ void CalcPartialA(int col, T d, const T* rr, T* a) {
         v0 = ss3; v1 = ss4; v2 = ss5;
     }
     T n = v0 * v0 + v1 * v1 + v2 * v2;
-    n = (n > eps) ? (T)1 / t_sqrt(n) : (T)0;
+    n = (n > eps) ? t_rcp(t_sqrt_pos(n)) : (T)0;
     a[col] = v0 * n; a[col + 3] = v1 * n; a[col + 6] = v2 * n;
 }
 // Completion of a unit vector x orthogonal to y when x has degenerated
@@ -132,7 +158,7 @@ __device__ __forceinline__ bool CalcCompleteA(T e0, T e1, T e2, T* a) {
     x1 -= d * y1; p += x1 * x1;
     x2 -= d * y2; p += x2 * x2;
     if (p > (T)TFMTOL) {
-        p = (T)1 / t_sqrt(p);
+        p = t_rcp(t_sqrt_pos(p));
         x0 *= p; x1 *= p; x2 *= p;
     } else if (!complete_orthogonal(y0, y1, y2, x0, x1, x2)) {
         return false;
@@ -152,13 +178,13 @@ __device__ __forceinline__ bool CalcRotMtx(const T* a, T* b) {
     b[0] = r0 * a[0] + b[1] * a[3] + b[2] * a[6]; d += b[0] * b[0];
     b[3] = r1 * a[0] + b[4] * a[3] + b[5] * a[6]; d += b[3] * b[3];
     b[6] = r2 * a[0] + b[7] * a[3] + b[8] * a[6]; d += b[6] * b[6];
-    d = (d > eps) ? (T)1 / t_sqrt(d) : (T)0;
+    d = (d > eps) ? t_rcp(t_sqrt_pos(d)) : (T)0;
     b[0] *= d; b[3] *= d; b[6] *= d;
     d = 0;
     b[1] = r0 * a[1] + b[1] * a[4] + b[2] * a[7]; d += b[1] * b[1];
     b[4] = r1 * a[1] + b[4] * a[4] + b[5] * a[7]; d += b[4] * b[4];
     b[7] = r2 * a[1] + b[7] * a[4] + b[8] * a[7]; d += b[7] * b[7];
-    d = (d > eps) ? (T)1 / t_sqrt(d) : (T)0;
+    d = (d > eps) ? t_rcp(t_sqrt_pos(d)) : (T)0;
     b[1] *= d; b[4] *= d; b[7] *= d;
     d = b[0] * b[1] + b[3] * b[4] + b[6] * b[7];
     T p = 0;
@@ -166,7 +192,7 @@ __device__ __forceinline__ bool CalcRotMtx(const T* a, T* b) {
     b[4] -= d * b[3]; p += b[4] * b[4];
     b[7] -= d * b[6]; p += b[7] * b[7];
     if (p > (T)TFMTOL) {
-        p = (T)1 / t_sqrt(p);
+        p = t_rcp(t_sqrt_pos(p));
         b[1] *= p; b[4] *= p; b[7] *= p;
     } else {
         T x0, x1, x2;
@@ -207,12 +233,18 @@ __device__ __forceinline__ void kabsch(const T* ccin, T n, bool dinv, float* tfm
         for (int i = 0; i < 3; i++) { t = c[CVq0 + i]; c[CVq0 + i] = c[CVr0 + i]; c[CVr0 + i] = t; }
     }
     T a[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1}, rr[6];
-    for (int i = CVq0; i < CVq0 + 3; i++) c[i] /= n;
+    const T yn = t_rcp(n);
+    for (int i = CVq0; i < CVq0 + 3; i++) c[i] = t_div(c[i], n, yn);
     CalcRmatrix(c);
-    for (int i = CVr0; i < CVr0 + 3; i++) c[i] /= n;
+    for (int i = CVr0; i < CVr0 + 3; i++) c[i] = t_div(c[i], n, yn);
     T scale = (t_abs(c[0]) + t_abs(c[1]) + t_abs(c[2]) + t_abs(c[3]) + t_abs(c[4]) + t_abs(c[5]) +
                t_abs(c[6]) + t_abs(c[7]) + t_abs(c[8])) * (T)(1.0f / 9.0f);
-    for (int i = 0; i < 9; i++) c[i] /= scale;
+    if (scale > (T)1e-18f && scale < (T)1e18f) {
+        const T ys = t_rcp(scale);
+        for (int i = 0; i < 9; i++) c[i] = t_div(c[i], scale, ys);
+    } else {
+        for (int i = 0; i < 9; i++) c[i] /= scale;
+    }
     T det = CalcDet(c);
     CalcRTR(c, rr);
     const T third = (T)(1.0f / 3.0f);

@@ -104,21 +104,20 @@ __device__ __forceinline__ int wq_next_block(const WorkQ& wq, int* slot) {
 
 // convergence of the covariance record (CheckConvergenceRefined_Complete,
 // MpStageBase.h:262-277): all 16 fields changed by less than 1e-5 relative
+__device__ __forceinline__ bool field_converged(float a, float b) {
+    // the smaller magnitude as a median with -inf: no canonicalisation as fminf has
+    const float m = __builtin_amdgcn_fmed3f(fabsf(a), fabsf(b), -__builtin_inff());
+    return fabsf(a - b) < m * RM_CONVEPSILON;
+}
+__device__ __forceinline__ bool field_converged(double a, double b) {
+    return fabs(a - b) < (fabs(a) < fabs(b) ? fabs(a) : fabs(b)) * (double)RM_CONVEPSILON;
+}
 template <typename T>
 __device__ __forceinline__ bool cc_converged(const T* a, T na, const T* b, T nb) {
-    int n = 0;
+    bool all = field_converged(na, nb);
 #pragma unroll
-    for (int f = 0; f < 15; f++) {
-        T d = a[f] - b[f];
-        T m = t_abs(a[f]) < t_abs(b[f]) ? t_abs(a[f]) : t_abs(b[f]);
-        if (t_abs(d) < m * (T)RM_CONVEPSILON) n++;
-    }
-    {
-        T d = na - nb;
-        T m = t_abs(na) < t_abs(nb) ? t_abs(na) : t_abs(nb);
-        if (t_abs(d) < m * (T)RM_CONVEPSILON) n++;
-    }
-    return n >= 16;
+    for (int f = 0; f < 15; f++) all &= field_converged(a[f], b[f]);
+    return all;
 }
 
 // ============================================================================
