@@ -14,7 +14,7 @@ import os
 import numpy as np
 
 from .capi import (ChunkView, Options, Results, STATUS, GTA_ALN_NFIELDS, GTA_TFM_NFIELDS,
-                   default_options)
+                   alignment_section_size, default_options)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libgta_amd.so")
 _lib = None
@@ -49,6 +49,8 @@ def lib():
         L.gta_set_references.restype = C.c_int
         L.gta_process.argtypes = [C.c_void_p, C.POINTER(Results)]
         L.gta_process.restype = C.c_int
+        L.gta_process_into.argtypes = [C.c_void_p, C.c_size_t] + [C.c_void_p] * 3 + [C.c_size_t, C.POINTER(Results)]
+        L.gta_process_into.restype = C.c_int
         L.gta_process_resident.argtypes = [C.c_void_p, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         L.gta_process_resident.restype = C.c_int
         L.gta_last_error.argtypes = [C.c_void_p]
@@ -87,19 +89,24 @@ def lib():
 
 
 class BlockResults:
-    """Host copy of the three result sections of one ProcessBlock."""
+    """Host copy of the three result sections of one ProcessBlock.  Without
+    `arrays` (the section arrays that `res` points to) the sections are copied
+    from the context's memory."""
 
-    def __init__(self, res):
+    def __init__(self, res, arrays=None):
         nq, nr = res.nqrys, res.nrefs
         self.nq, self.nr = nq, nr
-        self.alndata = np.ctypeslib.as_array(res.alndata, (nq * nr * GTA_ALN_NFIELDS,)).copy() \
-            .reshape(nq, nr, GTA_ALN_NFIELDS)
-        self.tfms = np.ctypeslib.as_array(res.tfms, (nq * nr * GTA_TFM_NFIELDS,)).copy() \
-            .reshape(nq, nr, GTA_TFM_NFIELDS)
-        # the alignment section can exceed 2 GiB (C.string_at takes an int size)
-        n = int(res.alnsize)
-        self.alns = (np.ctypeslib.as_array(C.cast(res.alns, C.POINTER(C.c_uint8)), (n,)).copy() if n
-                     else np.zeros(0, np.uint8))
+        if arrays is not None:
+            self.alndata, self.tfms, self.alns = arrays
+        else:
+            self.alndata = np.ctypeslib.as_array(res.alndata, (nq * nr * GTA_ALN_NFIELDS,)).copy() \
+                .reshape(nq, nr, GTA_ALN_NFIELDS)
+            self.tfms = np.ctypeslib.as_array(res.tfms, (nq * nr * GTA_TFM_NFIELDS,)).copy() \
+                .reshape(nq, nr, GTA_TFM_NFIELDS)
+            # the alignment section can exceed 2 GiB (C.string_at takes an int size)
+            n = int(res.alnsize)
+            self.alns = (np.ctypeslib.as_array(C.cast(res.alns, C.POINTER(C.c_uint8)), (n,)).copy() if n
+                         else np.zeros(0, np.uint8))
         self.seconds = res.seconds
         self.cells = res.dp_cells
 
@@ -130,8 +137,17 @@ class GtaBatch:
 
     def ProcessBlock(self):
         res = Results()
-        self._check(lib().gta_process(self._h, C.byref(res)))
-        return BlockResults(res)
+        if self._q is None or self._r is None:
+            self._check(lib().gta_process(self._h, C.byref(res)))
+            return BlockResults(res)
+        # straight into the arrays handed out; the alignment section is mostly
+        # zeros, and its zero pages are never touched
+        nq, nr = self._q.nstrs, self._r.nstrs
+        arrays = (np.empty((nq, nr, GTA_ALN_NFIELDS), np.float32), np.empty((nq, nr, GTA_TFM_NFIELDS), np.float32),
+                  np.zeros(alignment_section_size(nq, self._q.nposs, nr, self._r.nposs), np.uint8))
+        self._check(lib().gta_process_into(self._h, nq * nr, *(a.ctypes.data for a in arrays), arrays[2].size,
+                                           C.byref(res)))
+        return BlockResults(res, arrays)
 
     def process_resident(self):
         """Run the stage leaving results in HBM; returns (device seconds, DP cells)."""

@@ -109,6 +109,21 @@ struct DevState {
     unsigned long long* algflops;  // algorithmic FP32 operations per kernel class
 };
 
+// a pair with alignment rows: its packed rows are 5 x cols bytes from off on
+struct RowRec {
+    int pair, cols;
+    unsigned long long off;
+};
+// byte offset of pair p's first alignment row, and the distance between its
+// rows (production_match2aln.cu:130-133)
+__host__ __device__ inline size_t aln_row(const int* qlen, const unsigned* qdst, const unsigned* rdst, int rnposs,
+                                          int nr, int p, size_t& stride) {
+    const int qi = p / nr, ri = p % nr;
+    stride = (size_t)rnposs + (size_t)nr * (size_t)(qlen[qi] + 1);
+    return ((size_t)qi * rnposs + (size_t)nr * ((size_t)qdst[qi] + qi)) * 5 + (size_t)rdst[ri] +
+           (size_t)ri * (size_t)(qlen[qi] + 1);
+}
+
 // kernel classes for the measurement counters
 enum { KC_SECSTR = 0, KC_INIT, KC_FINDFRAG, KC_REFINE_GAPLESS, KC_DP, KC_REFINE_DP, KC_REFINE_FIN,
        KC_PROD_ALN, KC_MISC, KC_COUNT };

@@ -2043,10 +2043,8 @@ __device__ void prod_aln_pair(const DevChunk& Q, const DevChunk& R, const DevSta
     const float* ad2 = S.aln + base + 6 * S.alnplane;
     const float* aqp = ad2 + S.alnplane;
     const float* arp = aqp + S.alnplane;
-    const size_t alnofff = ((size_t)qi * R.nposs + (size_t)S.nr * (size_t)(qd + qi)) * 5;
-    const size_t dbalnlen = (size_t)R.nposs + (size_t)S.nr * (size_t)(qlen + 1);
-    const size_t dbalnbeg = (size_t)rd + (size_t)ri * (size_t)(qlen + 1);
-    char* row0 = alns + alnofff + dbalnbeg;
+    size_t dbalnlen;
+    char* row0 = alns + aln_row(Q.len, Q.dst, R.dst, R.nposs, S.nr, p, dbalnlen);
     auto put = [&](int col, char a, char mid, char b, char sa, char sb) {
         row0[col] = a; row0[dbalnlen + col] = mid; row0[2 * dbalnlen + col] = b;
         row0[3 * dbalnlen + col] = sa; row0[4 * dbalnlen + col] = sb;
@@ -2100,6 +2098,44 @@ __global__ __launch_bounds__(GTA_WAVE) void k_prod_aln(DevChunk Q, DevChunk R, D
     } else {
         prod_aln_pair(Q, R, S, alns, nodel, (int)blockIdx.x);
     }
+}
+
+// ============================================================================
+// The alignment section is a few thousand alignments in a space for every
+// pair's longest one, zeros otherwise.  The pairs with alignment rows are
+// listed (in any order) and their rows packed, so that the host copies what was
+// written: of a 16 x 12,000 search 6 of 350 MB.
+__global__ __launch_bounds__(256) void k_list_rows(DevState S, unsigned long long* tot, RowRec* recs) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x, lane = lane_id();
+    int n = 0;
+    if (p < S.nq * S.nr && !(S.flags[p] & CONV_LOWTMSC)) n = (int)S.out[(size_t)p * 15 + 4];
+    const unsigned long long m = __ballot(n > 0);
+    if (!m) return;
+    unsigned long long bytes = 5ull * n;        // inclusive sum over the wave's lanes
+#pragma unroll
+    for (int o = 1; o < GTA_WAVE; o <<= 1) {
+        const unsigned long long v = __shfl_up(bytes, o, GTA_WAVE);
+        if (lane >= o) bytes += v;
+    }
+    unsigned long long slot0 = 0, off0 = 0;
+    if (lane == GTA_WAVE - 1) {
+        slot0 = atomicAdd(tot, (unsigned long long)__popcll(m));
+        off0 = atomicAdd(tot + 1, bytes);
+    }
+    slot0 = __shfl(slot0, GTA_WAVE - 1, GTA_WAVE);
+    off0 = __shfl(off0, GTA_WAVE - 1, GTA_WAVE);
+    if (n > 0)
+        recs[slot0 + __popcll(m & ((1ull << lane) - 1ull))] = RowRec{p, n, off0 + bytes - 5ull * n};
+}
+// one wave per listed pair
+__global__ __launch_bounds__(GTA_WAVE) void k_pack_rows(DevChunk Q, DevChunk R, DevState S, const char* alns,
+                                                        const RowRec* recs, char* packed) {
+    const RowRec rec = recs[blockIdx.x];
+    size_t stride;
+    const char* row = alns + aln_row(Q.len, Q.dst, R.dst, R.nposs, S.nr, rec.pair, stride);
+    for (int r = 0; r < 5; r++)
+        for (int j = lane_id(); j < rec.cols; j += GTA_WAVE)
+            packed[rec.off + (size_t)r * rec.cols + j] = row[r * stride + j];
 }
 
 // ============================================================================
@@ -2631,6 +2667,17 @@ hipError_t launch_prod_aln(const DevChunk& Q, const DevChunk& R, const DevState&
                            const WorkQ& wq, int pgrid, hipStream_t st) {
     const int n = wq.items ? pgrid : S.nq * S.nr;
     hipLaunchKernelGGL(k_prod_aln, dim3(n), dim3(GTA_WAVE), 0, st, Q, R, S, alns, nodel, wq);
+    return hipGetLastError();
+}
+hipError_t launch_list_rows(const DevState& S, unsigned long long* tot, RowRec* recs, hipStream_t st) {
+    const long long np = (long long)S.nq * S.nr;
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, (int*)tot, 0, (size_t)4);
+    hipLaunchKernelGGL(k_list_rows, dim3(blocks_for(np, 256)), dim3(256), 0, st, S, tot, recs);
+    return hipGetLastError();
+}
+hipError_t launch_pack_rows(const DevChunk& Q, const DevChunk& R, const DevState& S, const char* alns,
+                            const RowRec* recs, size_t n, char* packed, hipStream_t st) {
+    if (n) hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)n), dim3(GTA_WAVE), 0, st, Q, R, S, alns, recs, packed);
     return hipGetLastError();
 }
 hipError_t launch_live_lists(const DevState& S, const unsigned char* bigmask, int* cnt, int* totals, int* lista,

@@ -103,6 +103,11 @@ hipError_t launch_prod_aln(const DevChunk& Q, const DevChunk& R, const DevState&
 // pass; cnt holds 3 ints per 1024 pairs, totals 3 ints
 hipError_t launch_live_lists(const DevState& S, const unsigned char* bigmask, int* cnt, int* totals, int* lista,
                              int* listb, int* listc, hipStream_t st);
+// the pairs with alignment rows (tot: their number and packed bytes), and
+// their rows packed
+hipError_t launch_list_rows(const DevState& S, unsigned long long* tot, RowRec* recs, hipStream_t st);
+hipError_t launch_pack_rows(const DevChunk& Q, const DevChunk& R, const DevState& S, const char* alns,
+                            const RowRec* recs, size_t n, char* packed, hipStream_t st);
 hipError_t launch_fill_i32(int* d, int v, size_t n, hipStream_t st);
 // mixed precision: RMSD of every output pair's final alignment from FP64 sums
 // and the quaternion matrix's largest eigenvalue (after the PROD1 refinement)

@@ -167,6 +167,14 @@ int gta_set_references(gta_ctx* ctx, const gta_chunk_view* refs);
  * result sections to host memory owned by ctx. */
 int gta_process(gta_ctx* ctx, gta_results* out);
 
+/* gta_process with the results in the caller's buffers: alndata for
+ * pairs >= nq*nr records of 15 floats, tfms for as many transforms of 12, alns
+ * at least gta_alignment_section_size() bytes, all zero on entry (fresh zero
+ * pages cost nothing: only the rows of aligned pairs are written where they
+ * are a small part of the section).  out's pointers are the caller's. */
+int gta_process_into(gta_ctx* ctx, size_t pairs, float* alndata, float* tfms, char* alns, size_t alns_bytes,
+                     gta_results* out);
+
 /* ---- stage without device allocation --------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory during a call (serving loops, harnesses that forbid hipMalloc):
@@ -223,8 +231,8 @@ int gta_dp_cell_counts(const gta_ctx* ctx, double* useful, double* launched);
  * Each pair's DP fill runs as one wave, as one workgroup of 4, 8 or 16 waves,
  * or pipelined over the whole device.  Off (the default), large pairs take
  * the grid form when they number at most half the compute units and the
- * W-wave form otherwise, and small chunks the W-wave form.  On, pairs of >= 4 strips of 64 rows and >= 2^18
- * cells are grouped by length bucket (log2 of the strip count, log2 of the
+ * W-wave form otherwise, and small chunks the W-wave form.  On, pairs of >= 4
+ * strips of 64 rows and >= 2^18 cells are grouped by length bucket (log2 of the strip count, log2 of the
  * reference length, log2 of the bucket's pair count); at the first
  * gta_process on a chunk pair, each bucket without a cached choice is timed
  * over the candidate forms (whole-chunk fills, identity superpositions) and
