@@ -137,7 +137,7 @@ struct gta_ctx {
     ChunkDev q, r;
     bool have_q = false, have_r = false;
     // pair state
-    DevBuf s_flags, s_grand, s_best0, s_prev, s_naln, s_qpos, s_rpos, s_fndx, s_fpos;
+    DevBuf s_flags, s_grand, s_best0, s_prev, s_naln, s_same, s_qpos, s_rpos, s_fndx, s_fpos;
     DevBuf s_tibest, s_tgrand, s_out, s_aln, s_btck, s_btckoff, s_rowbuf, s_cells, s_alns, s_algb;
     // DP forms: pair lists, and the rows, row offsets, first strips and item
     // counter of the device-wide fill
@@ -310,7 +310,7 @@ static std::vector<DevBuf*> all_bufs(gta_ctx* c) {
     return {&c->q.b_len, &c->q.b_dst, &c->q.b_na, &c->q.b_x, &c->q.b_y, &c->q.b_z, &c->q.b_rsd, &c->q.b_ss,
             &c->q.b_napos, &c->r.b_len, &c->r.b_dst, &c->r.b_na, &c->r.b_x, &c->r.b_y, &c->r.b_z,
             &c->r.b_rsd, &c->r.b_ss, &c->r.b_napos,
-            &c->s_flags, &c->s_grand, &c->s_best0, &c->s_prev, &c->s_naln, &c->s_qpos,
+            &c->s_flags, &c->s_grand, &c->s_best0, &c->s_prev, &c->s_naln, &c->s_same, &c->s_qpos,
             &c->s_rpos, &c->s_fndx, &c->s_fpos, &c->s_tibest, &c->s_tgrand, &c->s_out,
             &c->s_aln, &c->s_btck, &c->s_btckoff, &c->s_rowbuf, &c->s_cells, &c->s_alns,
             &c->s_algb, &c->s_dpbig, &c->s_grows, &c->s_growoff, &c->s_fail,
@@ -668,6 +668,7 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
     HIPCHK(c, c->s_best0.ensure(np * 4));
     HIPCHK(c, c->s_prev.ensure(np * 4));
     HIPCHK(c, c->s_naln.ensure(np * 4));
+    HIPCHK(c, c->s_same.ensure(np * 4));
     HIPCHK(c, c->s_qpos.ensure(np * 4));
     HIPCHK(c, c->s_rpos.ensure(np * 4));
     HIPCHK(c, c->s_fndx.ensure(np * 4));
@@ -698,7 +699,7 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
 
     S.nq = nq; S.nr = nr;
     S.flags = c->s_flags.as<int>(); S.grand = c->s_grand.as<float>(); S.best0 = c->s_best0.as<float>();
-    S.prevbest0 = c->s_prev.as<float>(); S.nalnposs = c->s_naln.as<int>();
+    S.prevbest0 = c->s_prev.as<float>(); S.nalnposs = c->s_naln.as<int>(); S.same = c->s_same.as<int>();
     S.qrypos = c->s_qpos.as<int>(); S.rfnpos = c->s_rpos.as<int>();
     S.sfragndx = c->s_fndx.as<int>(); S.sfragpos = c->s_fpos.as<int>();
     S.tfm_ibest = c->s_tibest.as<float>(); S.tfm_grand = c->s_tgrand.as<float>();

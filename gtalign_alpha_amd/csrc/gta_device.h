@@ -90,6 +90,7 @@ struct DevState {
     float* best0;
     float* prevbest0;
     int* nalnposs;
+    int* same;              // the last walk gave the alignment that the pair held before
     int* qrypos;
     int* rfnpos;
     int* sfragndx;

@@ -207,7 +207,7 @@ __global__ void k_init(DevChunk Q, DevChunk R, DevState S) {
     const int qi = pair_q(S, p), ri = pair_r(S, p);
     S.flags[p] = (Q.na[qi] == R.na[ri]) ? 0 : CONV_LOWTMSC;
     S.grand[p] = 0.f; S.best0[p] = 0.f; S.prevbest0[p] = 0.f;
-    S.nalnposs[p] = 0; S.qrypos[p] = 0; S.rfnpos[p] = 0; S.sfragndx[p] = 0; S.sfragpos[p] = 0;
+    S.nalnposs[p] = 0; S.same[p] = 0; S.qrypos[p] = 0; S.rfnpos[p] = 0; S.sfragndx[p] = 0; S.sfragpos[p] = 0;
     for (int i = 0; i < 12; i++) {
         float v = (i == 0 || i == 4 || i == 8) ? 1.f : 0.f;
         S.tfm_ibest[p * 12 + i] = v;
@@ -1137,6 +1137,9 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
     const bool constrained = prm.mode == DPM_CONSTRAINED;
     const float d82 = GetD82(Lq, Lr);
     int y0 = Lq - 1, x0 = Lr - 1, k = 0;
+    // the alignment that the pair holds, to see whether this one is the same
+    const int held = S.nalnposs[p];
+    bool same = true;
     int ym = 0, xm = -1;        // the lane's matched row and column of the last window
     for (;;) {
         const bool more = y0 >= 0 && x0 >= 0;
@@ -1165,6 +1168,7 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
             const unsigned long long km = __ballot(keep);
             if (keep) {
                 const int o = k + __popcll(km & ((1ull << lane) - 1ull));
+                if (o < held) same = same && aqp[o] == (float)ym && arp[o] == (float)xm;
                 aqx[o] = qx; aqy[o] = qy; aqz[o] = qz;
                 arx[o] = rx; ary[o] = ry; arz[o] = rz;
                 aqp[o] = (float)ym; arp[o] = (float)xm;
@@ -1219,7 +1223,11 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
         y0 -= l;
         x0 += f - 31 - l;
     }
-    if (lane == 0) S.nalnposs[p] = k;
+    same = __all(same) && k == held && k > 0;
+    if (lane == 0) {
+        S.nalnposs[p] = k;
+        S.same[p] = same;
+    }
 }
 
 __device__ __forceinline__ void dp_count(const DevState& S, const DpPair& P) {
@@ -1685,6 +1693,21 @@ __device__ __forceinline__ float gscore_cc_dp(const A& a, int L, const float* tf
     return s;
 }
 
+// DPRefine bookkeeping after a pair's refinement (MpStage1.cpp:455-510)
+__device__ __forceinline__ void dprefine_flags(const DevState& S, const RefineParams& prm, int p, int minlen) {
+    if (!prm.epi) return;
+    int fl = S.flags[p];
+    if (0 < prm.dpi && !(fl & (CONV_SCOREDP | CONV_LOWTMSC)) &&
+        fabsf(S.best0[p] - S.prevbest0[p]) < SCORE_CONVEPSILON)
+        fl |= CONV_SCOREDP;
+    if (prm.dpi + 1 < prm.maxndpiters && !(fl & (CONV_SCOREDP | CONV_LOWTMSC))) S.prevbest0[p] = S.best0[p];
+    if (prm.maxndpiters <= prm.dpi + 1) {
+        if (0.0f < prm.prescore && S.grand[p] < prm.prescore * (float)minlen) fl |= CONV_LOWTMSC;
+        fl &= ~CONV_SCOREDP;
+    }
+    S.flags[p] = fl;
+}
+
 // Superposition refinement over the DP alignment, one workgroup per pair
 // (FragmentBasedDPAlignmentRefinement, FinalFragmentBasedDPAlignmentRefinement
 // Phase1/2, ProductionFragmentBasedDPAlignmentRefinementPhase1/2:
@@ -1719,18 +1742,7 @@ __device__ void refine_dp_epilogue(const DevChunk& Q, const DevChunk& R, const D
             copy12(tg, b.tfm);
         }
     }
-    if (MODE == RM_DPREFINE && prm.epi) {
-        int fl = S.flags[p];
-        if (0 < prm.dpi && !(fl & (CONV_SCOREDP | CONV_LOWTMSC)) &&
-            fabsf(S.best0[p] - S.prevbest0[p]) < SCORE_CONVEPSILON)
-            fl |= CONV_SCOREDP;
-        if (prm.dpi + 1 < prm.maxndpiters && !(fl & (CONV_SCOREDP | CONV_LOWTMSC))) S.prevbest0[p] = S.best0[p];
-        if (prm.maxndpiters <= prm.dpi + 1) {
-            if (0.0f < prm.prescore && S.grand[p] < prm.prescore * (float)min(qlen, rlen)) fl |= CONV_LOWTMSC;
-            fl &= ~CONV_SCOREDP;
-        }
-        S.flags[p] = fl;
-    }
+    if (MODE == RM_DPREFINE) dprefine_flags(S, prm, p, min(qlen, rlen));
 }
 
 // LDS of a refinement workgroup of W waves (W * NGW slot groups)
@@ -1762,6 +1774,14 @@ __device__ void refine_pair(const DevChunk& Q, const DevChunk& R, const DevState
     if (MODE == RM_DPREFINE) skip = flags != 0;
     else skip = (flags & CONV_LOWTMSC) != 0;
     if (skip && MODE != RM_DPREFINE) return;
+    if (MODE == RM_DPREFINE && !skip && S.same[p]) {
+        // The slots start from fragments of the alignment and use no earlier
+        // superposition, so the refinement of an unchanged alignment repeats
+        // the last one, whose best score and transform the pair still holds
+        // (1 of 16 refinements of a 16 x 12,000 search, 1 of 5 of a 1 x 256 one).
+        if (threadIdx.x == 0 && !parts) dprefine_flags(S, prm, p, min(qlen, rlen));
+        return;
+    }
 
     const int L = skip ? 0 : S.nalnposs[p];
     const size_t base = (size_t)qi * (size_t)R.nposs + (size_t)R.dst[ri];
@@ -2446,6 +2466,11 @@ __global__ void k_merge_parts(DevChunk Q, DevChunk R, DevState S, RefineParams p
         return;
     }
     if (KIND == 2 && MODE != RM_DPREFINE && (flags & CONV_LOWTMSC)) return;
+    if (KIND == 2 && MODE == RM_DPREFINE && flags == 0 && S.same[p]) {
+        // no part ran (refine_pair)
+        dprefine_flags(S, prm, p, min(Q.len[pair_q(S, p)], R.len[pair_r(S, p)]));
+        return;
+    }
     SlotBest b = parts[(size_t)i * nparts];
     for (int k = 1; k < nparts; k++) {
         const SlotBest& c = parts[(size_t)i * nparts + k];
