@@ -1779,6 +1779,10 @@ __device__ void refine_pair(const DevChunk& Q, const DevChunk& R, const DevState
         // superposition, so the refinement of an unchanged alignment repeats
         // the last one, whose best score and transform the pair still holds
         // (1 of 16 refinements of a 16 x 12,000 search, 1 of 5 of a 1 x 256 one).
+        // Every wave has read the pair's flags before they change: a wave that
+        // read them later would take the other way out of this function, with
+        // more barriers than the rest of its workgroup.
+        __syncthreads();
         if (threadIdx.x == 0 && !parts) dprefine_flags(S, prm, p, min(qlen, rlen));
         return;
     }
