@@ -137,7 +137,7 @@ struct gta_ctx {
     ChunkDev q, r;
     bool have_q = false, have_r = false;
     // pair state
-    DevBuf s_flags, s_grand, s_best0, s_prev, s_naln, s_same, s_qpos, s_rpos, s_fndx, s_fpos;
+    DevBuf s_flags, s_grand, s_best0, s_prev, s_naln, s_qpos, s_rpos, s_fndx, s_fpos;
     DevBuf s_tibest, s_tgrand, s_out, s_aln, s_btck, s_btckoff, s_rowbuf, s_cells, s_alns, s_algb;
     // DP forms: pair lists, and the rows, row offsets, first strips and item
     // counter of the device-wide fill
@@ -310,7 +310,7 @@ static std::vector<DevBuf*> all_bufs(gta_ctx* c) {
     return {&c->q.b_len, &c->q.b_dst, &c->q.b_na, &c->q.b_x, &c->q.b_y, &c->q.b_z, &c->q.b_rsd, &c->q.b_ss,
             &c->q.b_napos, &c->r.b_len, &c->r.b_dst, &c->r.b_na, &c->r.b_x, &c->r.b_y, &c->r.b_z,
             &c->r.b_rsd, &c->r.b_ss, &c->r.b_napos,
-            &c->s_flags, &c->s_grand, &c->s_best0, &c->s_prev, &c->s_naln, &c->s_same, &c->s_qpos,
+            &c->s_flags, &c->s_grand, &c->s_best0, &c->s_prev, &c->s_naln, &c->s_qpos,
             &c->s_rpos, &c->s_fndx, &c->s_fpos, &c->s_tibest, &c->s_tgrand, &c->s_out,
             &c->s_aln, &c->s_btck, &c->s_btckoff, &c->s_rowbuf, &c->s_cells, &c->s_alns,
             &c->s_algb, &c->s_dpbig, &c->s_grows, &c->s_growoff, &c->s_fail,
@@ -426,10 +426,10 @@ static Geom make_geom(const gta_ctx* c) {
 // ---- DP launch forms ----------------------------------------------------------
 // Every pair's fill runs in one of five forms: one wave (k_dp), one workgroup
 // of 4, 8 or 16 waves (k_dp_mw) or the device-wide strip pipeline
-// (k_dp_grid).  By default large pairs (Lq*Lr >= mw_min_cells, >= mw_min_strips
+// (k_dp's grid pairs).  By default large pairs (Lq*Lr >= mw_min_cells, >= mw_min_strips
 // groups of 64 rows, Lr >= 256) that number at most half the CUs take the grid
-// form, and the others one wave or, in a small chunk, one workgroup
-// (default_dp_forms); gta_test_set_dp_buckets puts the large ones into a
+// form, and of the others the longest may take one workgroup (in a small chunk)
+// or the grid form (default_dp_forms); gta_test_set_dp_buckets puts the large ones into a
 // workgroup and the others into one wave instead.  With autotuning on, pairs
 // of >= 4 groups and >= 2^18 cells are grouped by length bucket (log2 of the
 // groups, log2 of Lr, log2 of the bucket's pair count) and each bucket's form
@@ -487,7 +487,7 @@ static int upload_dp_buckets(gta_ctx* c, const std::vector<unsigned char>& form,
     HIPCHK(c, c->s_growoff.ensure(offs.size() * 8));
     HIPCHK(c, c->s_grows.ensure(rowtot * 4));
     HIPCHK(c, c->s_gstrip0.ensure(s0.size() * 4));
-    HIPCHK(c, c->s_gnext.ensure(4));
+    HIPCHK(c, c->s_gnext.ensure(((size_t)B.ngrid + 1) * 4));
     HIPCHK(c, hipMemcpy(c->s_growoff.p, offs.data(), offs.size() * 8, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->s_gstrip0.p, s0.data(), s0.size() * 4, hipMemcpyHostToDevice));
     B.gstrip0 = c->s_gstrip0.as<int>();
@@ -495,22 +495,28 @@ static int upload_dp_buckets(gta_ctx* c, const std::vector<unsigned char>& form,
     B.grows = c->s_grows.as<float>();
     B.growoff = c->s_growoff.as<unsigned long long>();
     B.growtot = rowtot;
-    B.gworkers = std::max(1, std::min(tot, 2 * c->ncu));
+    B.gworkers = std::max(1, std::min(tot, 8 * c->ncu));
     return GTA_OK;
 }
 
-// A chunk of at most two pairs per CU leaves most of the device idle, and its
-// launches last as long as the longest fill.  One wave takes 0.05 us per step
-// and row of a lane (measured: 65 us for 256 x 256, 0.23 ms for 500 x 500, 0.85
-// ms for 1,000 x 1,000 residues), one workgroup of W waves 0.08 us per step with
-// the strips 80 steps apart (45 us, 0.11 ms and, with 16 waves, 0.2 ms for the
-// same pairs): there, a pair that a workgroup fills in 3/4 of the time or less
-// takes the smallest workgroup that holds its strips.  In larger chunks one
-// wave per pair is faster on the whole (40,000 pairs of 256 x 256: 2.2 against
-// 4.0 ms, 1,600: 0.17 against 0.21 ms; the longest tenth in workgroups cost the
-// 30 fills of a 4 x 1,500 search 5 of 11 ms, as their launch follows the
-// other's).
-constexpr double DP_US_ROWSTEP = 0.05, DP_US_MWSTEP = 0.08;
+// One wave fills a pair in 0.05 us per step and row of a lane (measured: 65 us
+// for 256 x 256, 0.23 ms for 500 x 500, 0.85 ms for 1,000 x 1,000 residues),
+// several in 0.08 us per step with the strips 80 steps apart in a workgroup (45
+// us, 0.11 ms and, with 16 waves, 0.2 ms for the same pairs) and about 100 apart
+// in the grid form, at 1.8 times the device's time (40,000 pairs of 256 x 256:
+// 4.0 against 2.2 ms).  A pair that several waves fill in 3/4 of the time or
+// less
+//  - takes a workgroup that holds its strips in a chunk of at most two pairs
+//    per CU, which leaves most of the device idle;
+//  - takes the grid form in a larger chunk whose longest fill is longer than
+//    the device's share of all fills (3.6e-5 us per step and group of 64 rows;
+//    the prescreen leaves about a third of it), if it is one of the longest
+//    that make up a tenth of the share and longer than 0.1 ms: a launch then
+//    ends with shorter fills (30 fills of 400 residues against 25,000 chains
+//    of up to 4,000: 34.9 -> 27.7 ms, with seeds at every fifth diagonal 48 ->
+//    30; 4 x 1,500: 10.7 -> 8.1).  In a launch of its own behind the others, in
+//    workgroups, the same tenth cost the 4 x 1,500 fills 5 ms more.
+constexpr double DP_US_ROWSTEP = 0.05, DP_US_STEP = 0.08, DP_US_GROUP = 3.6e-5;
 
 static int dp_mw_form(int strips) { return strips <= 4 ? DPF_W4 : strips <= 8 ? DPF_W8 : DPF_W16; }
 
@@ -539,14 +545,58 @@ static void default_dp_forms(const gta_ctx* c, std::vector<unsigned char>& form)
     if (grid)
         for (int pidx : big) form[pidx] = DPF_GRID;
     if (c->dp_forced) return;
-    if ((long long)nq * nr > 2ll * c->ncu) return;
+    // these forms need lists and rows of their own: not at the end of the
+    // scratch of gta_process_noalloc
+    if (g_arena && g_arena->cap - std::min(g_arena->cap, g_arena->off) < (1u << 20)) return;
+    auto one_us = [](int G, int Lr) { return DP_US_ROWSTEP * G * (Lr + 63.0); };
+    if ((long long)nq * nr <= 2ll * c->ncu) {
+        for (int qi = 0; qi < nq; qi++) {
+            const int G = (c->q.len[qi] + 63) / 64, f = dp_mw_form(G), W = 4 << (f - DPF_W4);
+            for (int ri = 0; ri < nr; ri++) {
+                unsigned char& fm = form[(size_t)qi * nr + ri];
+                const int Lr = c->r.len[ri];
+                const double mw = DP_US_STEP * ((G + W - 1) / W) * (Lr + 63.0 + 80.0 * (std::min(W, G) - 1));
+                if (fm == DPF_ONE && mw <= 0.75 * one_us(G, Lr)) fm = (unsigned char)f;
+            }
+        }
+        return;
+    }
+    if (g_arena || c->dp_grid == 2) return;
+    // share of the device by class of one-wave time (4 classes an octave), over
+    // runs of equal reference lengths (the references are sorted by length)
+    constexpr int NB = 128;
+    std::vector<double> share(NB, 0.0);
+    const double scale = 1024.0 / (4.0 * c->ncu);
+    auto class_of = [](double us) { return std::min(NB - 1, std::max(0, (int)(4.0 * log2(us)))); };
+    auto eligible = [&](int G, int Lr) { return DP_US_STEP * (Lr + 63.0 + 100.0 * (G - 1)) <= 0.75 * one_us(G, Lr); };
+    std::vector<std::pair<int, int>> runs;      // (first reference, length)
+    for (int ri = 0; ri < nr; ri++)
+        if (runs.empty() || runs.back().second != c->r.len[ri]) runs.push_back({ri, c->r.len[ri]});
+    runs.push_back({nr, 0});
+    double total = 0.0, longest = 0.0;
     for (int qi = 0; qi < nq; qi++) {
-        const int G = (c->q.len[qi] + 63) / 64, f = dp_mw_form(G), W = 4 << (f - DPF_W4);
-        for (int ri = 0; ri < nr; ri++) {
-            unsigned char& fm = form[(size_t)qi * nr + ri];
-            const double steps = c->r.len[ri] + 63.0;
-            const double mw = DP_US_MWSTEP * ((G + W - 1) / W) * (steps + 80.0 * (std::min(W, G) - 1));
-            if (fm == DPF_ONE && mw <= 0.75 * DP_US_ROWSTEP * G * steps) fm = (unsigned char)f;
+        const int G = (c->q.len[qi] + 63) / 64;
+        for (size_t k = 0; k + 1 < runs.size(); k++) {
+            const int Lr = runs[k].second, n = runs[k + 1].first - runs[k].first;
+            const double us = n * DP_US_GROUP * scale * G * (Lr + 63.0);
+            total += us;
+            longest = std::max(longest, one_us(G, Lr));
+            if (eligible(G, Lr)) share[class_of(one_us(G, Lr))] += us;
+        }
+    }
+    if (longest <= (c->opts.prescore > 0.f ? 0.33 : 1.0) * total) return;
+    int th = NB;
+    double above = 0.0;
+    while (th > class_of(100.0) && above + share[th - 1] <= 0.1 * total) above += share[--th];
+    for (int qi = 0; qi < nq; qi++) {
+        const int G = (c->q.len[qi] + 63) / 64;
+        for (size_t k = 0; k + 1 < runs.size(); k++) {
+            const int Lr = runs[k].second;
+            if (class_of(one_us(G, Lr)) < th || !eligible(G, Lr)) continue;
+            for (int ri = runs[k].first; ri < runs[k + 1].first; ri++) {
+                unsigned char& fm = form[(size_t)qi * nr + ri];
+                if (fm == DPF_ONE) fm = DPF_GRID;
+            }
         }
     }
 }
@@ -668,7 +718,6 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
     HIPCHK(c, c->s_best0.ensure(np * 4));
     HIPCHK(c, c->s_prev.ensure(np * 4));
     HIPCHK(c, c->s_naln.ensure(np * 4));
-    HIPCHK(c, c->s_same.ensure(np * 4));
     HIPCHK(c, c->s_qpos.ensure(np * 4));
     HIPCHK(c, c->s_rpos.ensure(np * 4));
     HIPCHK(c, c->s_fndx.ensure(np * 4));
@@ -699,7 +748,7 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
 
     S.nq = nq; S.nr = nr;
     S.flags = c->s_flags.as<int>(); S.grand = c->s_grand.as<float>(); S.best0 = c->s_best0.as<float>();
-    S.prevbest0 = c->s_prev.as<float>(); S.nalnposs = c->s_naln.as<int>(); S.same = c->s_same.as<int>();
+    S.prevbest0 = c->s_prev.as<float>(); S.nalnposs = c->s_naln.as<int>(); S.same = c->s_fndx.as<int>();
     S.qrypos = c->s_qpos.as<int>(); S.rfnpos = c->s_rpos.as<int>();
     S.sfragndx = c->s_fndx.as<int>(); S.sfragpos = c->s_fpos.as<int>();
     S.tfm_ibest = c->s_tibest.as<float>(); S.tfm_grand = c->s_tgrand.as<float>();

@@ -90,7 +90,8 @@ struct DevState {
     float* best0;
     float* prevbest0;
     int* nalnposs;
-    int* same;              // the last walk gave the alignment that the pair held before
+    int* same;              // DPRefine: the last walk gave the alignment that the pair held before
+                            // (in sfragndx, which the final stage's first phase sets)
     int* qrypos;
     int* rfnpos;
     int* sfragndx;

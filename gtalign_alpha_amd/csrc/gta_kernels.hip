@@ -207,7 +207,7 @@ __global__ void k_init(DevChunk Q, DevChunk R, DevState S) {
     const int qi = pair_q(S, p), ri = pair_r(S, p);
     S.flags[p] = (Q.na[qi] == R.na[ri]) ? 0 : CONV_LOWTMSC;
     S.grand[p] = 0.f; S.best0[p] = 0.f; S.prevbest0[p] = 0.f;
-    S.nalnposs[p] = 0; S.same[p] = 0; S.qrypos[p] = 0; S.rfnpos[p] = 0; S.sfragndx[p] = 0; S.sfragpos[p] = 0;
+    S.nalnposs[p] = 0; S.qrypos[p] = 0; S.rfnpos[p] = 0; S.sfragndx[p] = 0; S.sfragpos[p] = 0;
     for (int i = 0; i < 12; i++) {
         float v = (i == 0 || i == 4 || i == 8) ? 1.f : 0.f;
         S.tfm_ibest[p * 12 + i] = v;
@@ -1226,7 +1226,7 @@ __device__ void dp_walk(const DevChunk& Q, const DevChunk& R, const DevState& S,
     same = __all(same) && k == held && k > 0;
     if (lane == 0) {
         S.nalnposs[p] = k;
-        S.same[p] = same;
+        if (!constrained) S.same[p] = same;
     }
 }
 
@@ -1265,20 +1265,123 @@ __device__ __forceinline__ void dp_pair(const DevChunk& Q, const DevChunk& R, co
     dp_walk(Q, R, S, prm, P, bt, DP_RM);
 }
 
-// One wave per pair: block b takes pair plist[b] (b without a list), or, with
-// a work queue, the waves of a persistent grid take queued pairs until the
-// queue is drained.
+// Row handoff between workgroups anywhere on the device (grid pairs): every
+// strip has its own row in HBM, filled with ROW_EMPTY (a NaN, which no cell
+// value is) before the launch, and a value itself says that it is there.  The
+// values are relaxed agent-scope atomics of 32 bits, so no fence, cache
+// write-back or counter stands between the store and the load; a strip loads
+// its 16 values a block ahead and again (bounded spin) until all are there.
+constexpr unsigned ROW_EMPTY = 0x7fc0e3d7u;
+struct RowGrid {
+    static constexpr bool IN_LDS = false;
+    const float* in;
+    float* out;
+    int* fail;      // set when a wait gave up; every other wait then gives up too
+    __device__ __forceinline__ float fetch(int c, int Lr) {
+        return (lane_id() < 16 && c < Lr) ? __hip_atomic_load(in + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                          : 0.f;
+    }
+    __device__ __forceinline__ bool take(float& v, int t0, int Lr) {
+        for (long long it = 0; __any(__float_as_uint(v) == ROW_EMPTY); it++) {
+            if (it > (1ll << 22) || __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                if (lane_id() == 0) __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return false;
+            }
+            v = fetch(t0 + lane_id(), Lr);
+        }
+        return true;
+    }
+    __device__ __forceinline__ bool put(int c, int, int Lr, float v) {
+        if (lane_id() >= 48 && c >= 0 && c < Lr)
+            __hip_atomic_store(out + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    }
+};
+
+// Grid pairs: long pairs whose strips (of one row group) are spread over
+// one-wave workgroups.  Workers take (pair, strip) items in increasing order
+// from a global counter; strip s waits on strip s-1's row (rows: ngroups x Lr
+// floats per pair at rowoff[k]; strip0[k] is pair k's first item).  Items are
+// handed out in order and a strip waits only on the strip before it, which a
+// running worker already holds, so the lowest unfinished strip never waits and
+// the fill always drains.  Same cells as the one-wave fill.  The worker that
+// finishes a pair's last strip (done[k] counts them, after a device-wide
+// release of the strip's codes) walks it.
+struct DpGrid {
+    const int* plist;
+    int npairs;
+    const int* strip0;
+    int* next;          // item counter, then done[npairs]
+    float* rows;
+    const unsigned long long* rowoff;
+    int* failflag;
+    int workers;
+};
+template <int SC, bool GAP0>
+__device__ __forceinline__ void dp_grid_items(const DevChunk& Q, const DevChunk& R, const DevState& S,
+                                              const DpParams& prm, const DpGrid& G, DpLds& lds) {
+    const int total = G.strip0[G.npairs];
+    for (;;) {
+        int item = 0;
+        if (lane_id() == 0) item = atomicAdd(G.next, 1);
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item >= total) break;
+        int lo = 0, hi = G.npairs - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (G.strip0[mid] <= item) lo = mid; else hi = mid - 1;
+        }
+        const int k = lo, s = item - G.strip0[k];
+        DpPair P;
+        if (!dp_setup(Q, R, S, prm, G.plist[k], P)) continue;
+        const int ngroups = G.strip0[k + 1] - G.strip0[k], nblk = (P.Lr + 63 + 15) >> 4;
+        float* prow = G.rows + G.rowoff[k];
+        unsigned* bt = S.btck + S.btckoff[P.p];
+        unsigned* sbt = bt + ((size_t)(s * nblk) << 6);
+        RowGrid io{s > 0 ? prow + (size_t)(s - 1) * P.Lr : nullptr, prow + (size_t)s * P.Lr, G.failflag};
+        const bool ok = s + 1 < ngroups
+                            ? dp_sweep<SC, GAP0, true, 1, true>(Q, R, prm, P, s, sbt, lds, io, nullptr, nullptr)
+                            : dp_sweep<SC, GAP0, true, 1, false>(Q, R, prm, P, s, sbt, lds, io, nullptr, nullptr);
+        if (!ok) {
+            if (lane_id() == 0) S.nalnposs[P.p] = 0;
+            break;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        int before = 0;
+        if (lane_id() == 0) before = atomicAdd(G.next + 1 + k, 1);
+        before = __builtin_amdgcn_readfirstlane(before);
+        if (before == ngroups - 1) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            dp_count(S, P);
+            dp_walk(Q, R, S, prm, P, bt, 1);
+        }
+    }
+}
+
+// Grid pairs alone, without k_dp's register bound: 30 fills of 6,007 x 6,007
+// residues 21.7 ms, in k_dp 24.2.
+template <int SC, bool GAP0>
+__global__ __launch_bounds__(GTA_WAVE) void k_dp_grid(DevChunk Q, DevChunk R, DevState S, DpParams prm, DpGrid G) {
+    __shared__ DpLds lds;
+    dp_grid_items<SC, GAP0>(Q, R, S, prm, G, lds);
+}
+
+// One wave per pair: behind the grid pairs' workers, block b takes pair
+// plist[b] (b without a list), or, with a work queue, the waves of a persistent
+// grid take grid items and then queued pairs until both are drained.
 template <int SC, bool GAP0>
 __global__ __launch_bounds__(GTA_WAVE) __attribute__((amdgpu_waves_per_eu(DP_WAVES))) void k_dp(
-    DevChunk Q, DevChunk R, DevState S, DpParams prm, const int* plist, WorkQ wq) {
+    DevChunk Q, DevChunk R, DevState S, DpParams prm, const int* plist, WorkQ wq, DpGrid G) {
     __shared__ DpLds lds;
     __shared__ float gtab[SC == SC_SSRR ? NGT * NGT : 1];
     if (SC == SC_SSRR) load_gtab(gtab, prm.rrw);
+    const int b = (int)blockIdx.x - G.workers;
+    if (SC != SC_SSRR && G.npairs && (b < 0 || wq.items)) dp_grid_items<SC, GAP0>(Q, R, S, prm, G, lds);
+    if (b < 0 && !wq.items) return;
     const int n = wq.items ? *wq.count : 0;
     int it = wq.items ? wq_next_wave(wq) : -1;
     while (it < n) {
-        dp_pair<SC, GAP0>(Q, R, S, prm, wq.items ? wq.items[it] : plist ? plist[blockIdx.x] : (int)blockIdx.x, lds,
-                          gtab);
+        dp_pair<SC, GAP0>(Q, R, S, prm, wq.items ? wq.items[it] : plist ? plist[b] : b, lds, gtab);
         if (!wq.items) break;
         it = wq_next_wave(wq);
     }
@@ -1463,90 +1566,6 @@ __global__ __launch_bounds__(W * GTA_WAVE) void k_dp_mw(DevChunk Q, DevChunk R, 
     }
     dp_count(S, P);
     if (w == 0) dp_walk(Q, R, S, prm, P, bt, MW_RM);
-}
-
-// Row handoff between workgroups anywhere on the device (k_dp_grid): every
-// strip has its own row in HBM, filled with ROW_EMPTY (a NaN, which no cell
-// value is) before the launch, and a value itself says that it is there.  The
-// values are relaxed agent-scope atomics of 32 bits, so no fence, cache
-// write-back or counter stands between the store and the load; a strip loads
-// its 16 values a block ahead and again (bounded spin) until all are there.
-constexpr unsigned ROW_EMPTY = 0x7fc0e3d7u;
-struct RowGrid {
-    static constexpr bool IN_LDS = false;
-    const float* in;
-    float* out;
-    int* fail;      // set when a wait gave up; every other wait then gives up too
-    __device__ __forceinline__ float fetch(int c, int Lr) {
-        return (lane_id() < 16 && c < Lr) ? __hip_atomic_load(in + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                          : 0.f;
-    }
-    __device__ __forceinline__ bool take(float& v, int t0, int Lr) {
-        for (long long it = 0; __any(__float_as_uint(v) == ROW_EMPTY); it++) {
-            if (it > (1ll << 22) || __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                if (lane_id() == 0) __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return false;
-            }
-            v = fetch(t0 + lane_id(), Lr);
-        }
-        return true;
-    }
-    __device__ __forceinline__ bool put(int c, int, int Lr, float v) {
-        if (lane_id() >= 48 && c >= 0 && c < Lr)
-            __hip_atomic_store(out + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return true;
-    }
-};
-
-// DP fill of a few very large pairs by the whole device: one-wave workgroups
-// take (pair, strip) items in increasing order from a global counter and sweep
-// them (strips of one row group; rows: ngroups x Lr floats per pair at
-// rowoff[k]; strip0[k] is pair k's first item).  Items are handed out in order
-// and a strip waits only on the strip before it, which a running workgroup
-// already holds, so the lowest unfinished strip never waits and the fill
-// always drains.  Same cells as k_dp; k_dp_grid_walk then walks each pair.
-template <int SC, bool GAP0>
-__global__ __launch_bounds__(GTA_WAVE) void k_dp_grid(DevChunk Q, DevChunk R, DevState S, DpParams prm,
-                                                       const int* plist, int npairs, const int* strip0,
-                                                       int* next, float* rows, const unsigned long long* rowoff,
-                                                       int* failflag) {
-    __shared__ DpLds lds;
-    const int total = strip0[npairs];
-    for (;;) {
-        int item = 0;
-        if (lane_id() == 0) item = atomicAdd(next, 1);
-        item = __builtin_amdgcn_readfirstlane(__shfl(item, 0, GTA_WAVE));
-        if (item >= total) break;
-        int lo = 0, hi = npairs - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (strip0[mid] <= item) lo = mid; else hi = mid - 1;
-        }
-        const int k = lo, s = item - strip0[k];
-        DpPair P;
-        if (!dp_setup(Q, R, S, prm, plist[k], P)) continue;
-        const int ngroups = strip0[k + 1] - strip0[k], nblk = (P.Lr + 63 + 15) >> 4;
-        float* prow = rows + rowoff[k];
-        unsigned* bt = S.btck + S.btckoff[P.p] + ((size_t)(s * nblk) << 6);
-        RowGrid io{s > 0 ? prow + (size_t)(s - 1) * P.Lr : nullptr, prow + (size_t)s * P.Lr, failflag};
-        const bool ok = s + 1 < ngroups
-                            ? dp_sweep<SC, GAP0, true, 1, true>(Q, R, prm, P, s, bt, lds, io, nullptr, nullptr)
-                            : dp_sweep<SC, GAP0, true, 1, false>(Q, R, prm, P, s, bt, lds, io, nullptr, nullptr);
-        if (!ok) break;
-    }
-}
-
-// backtrace walk of the pairs k_dp_grid filled (one wave per pair)
-__global__ __launch_bounds__(GTA_WAVE) void k_dp_grid_walk(DevChunk Q, DevChunk R, DevState S, DpParams prm,
-                                                            const int* plist, const int* failflag) {
-    DpPair P;
-    if (!dp_setup(Q, R, S, prm, plist[blockIdx.x], P)) return;
-    if (*failflag) {
-        if (threadIdx.x == 0) S.nalnposs[P.p] = 0;
-        return;
-    }
-    dp_count(S, P);
-    dp_walk(Q, R, S, prm, P, S.btck + S.btckoff[P.p], 1);
 }
 
 // ============================================================================
@@ -2571,9 +2590,33 @@ hipError_t launch_dp(const DevChunk& Q, const DevChunk& R, const DevState& S, co
         }                                                                   \
     } while (0)
     const int nsmall = wq.items ? pgrid : (B.small ? B.nsmall : S.nq * S.nr);
-    if (nsmall > 0) {
-#define GTA_K1(US, G0) \
-    hipLaunchKernelGGL((k_dp<US, G0>), dim3(nsmall), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.small, wq)
+    DpGrid G{};
+    if (B.ngrid > 0 && L.usess == SC_SSRR) {
+        // The SS/residue fill does not use the grid form: its grid-form run
+        // stalled on the GPU with no cause found yet.  Those pairs run as
+        // 4-wave workgroups instead.
+        hipLaunchKernelGGL((k_dp_mw<SC_SSRR, false, 4>), dim3(B.ngrid), dim3(4 * GTA_WAVE), 0, st, Q, R, S, prm,
+                           B.grid, B.failflag);
+    } else if (B.ngrid > 0) {
+        // every row empty and the counters at zero for every fill
+        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((long long)B.growtot, 256)), dim3(256), 0, st, (int*)B.grows,
+                           (int)ROW_EMPTY, B.growtot);
+        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((long long)B.ngrid + 1, 256)), dim3(256), 0, st, B.gnext, 0,
+                           (size_t)B.ngrid + 1);
+        G = DpGrid{B.grid, B.ngrid, B.gstrip0, B.gnext, B.grows, B.growoff, B.failflag, wq.items ? 0 : B.gworkers};
+    }
+    if (nsmall == 0 && G.workers > 0) {
+#define GTA_KG(US, G0) \
+    hipLaunchKernelGGL((k_dp_grid<US, G0>), dim3(G.workers), dim3(GTA_WAVE), 0, st, Q, R, S, prm, G)
+        if (L.usess == SC_TMSS) {
+            if (L.gap0) GTA_KG(SC_TMSS, true); else GTA_KG(SC_TMSS, false);
+        } else {
+            if (L.gap0) GTA_KG(SC_TM, true); else GTA_KG(SC_TM, false);
+        }
+#undef GTA_KG
+    } else if (nsmall > 0) {
+#define GTA_K1(US, G0)                                                                                           \
+    hipLaunchKernelGGL((k_dp<US, G0>), dim3(nsmall + G.workers), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.small, wq, G)
         GTA_DPV(GTA_K1);
 #undef GTA_K1
     }
@@ -2590,28 +2633,6 @@ hipError_t launch_dp(const DevChunk& Q, const DevChunk& R, const DevState& S, co
 #undef GTA_KMW8
 #undef GTA_KMW16
 #undef GTA_MW
-    if (B.ngrid > 0 && L.usess == SC_SSRR) {
-        // The SS/residue fill does not use the device-wide pipeline: its
-        // grid-form run stalled on the GPU with no cause found yet.  Those
-        // pairs run as 4-wave workgroups instead.
-        hipLaunchKernelGGL((k_dp_mw<SC_SSRR, false, 4>), dim3(B.ngrid), dim3(4 * GTA_WAVE), 0, st, Q, R, S, prm,
-                           B.grid, B.failflag);
-    } else if (B.ngrid > 0) {
-        // every row empty and the item counter at zero for every fill
-        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((long long)B.growtot, 256)), dim3(256), 0, st, (int*)B.grows,
-                           (int)ROW_EMPTY, B.growtot);
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, st, B.gnext, 0, (size_t)1);
-#define GTA_KG(US, G0)                                                                                    \
-    hipLaunchKernelGGL((k_dp_grid<US, G0>), dim3(B.gworkers), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.grid, \
-                       B.ngrid, B.gstrip0, B.gnext, B.grows, B.growoff, B.failflag)
-        if (L.usess == SC_TMSS) {
-            if (L.gap0) GTA_KG(SC_TMSS, true); else GTA_KG(SC_TMSS, false);
-        } else {
-            if (L.gap0) GTA_KG(SC_TM, true); else GTA_KG(SC_TM, false);
-        }
-#undef GTA_KG
-        hipLaunchKernelGGL(k_dp_grid_walk, dim3(B.ngrid), dim3(GTA_WAVE), 0, st, Q, R, S, prm, B.grid, B.failflag);
-    }
 #undef GTA_DPV
     return hipGetLastError();
 }

@@ -28,15 +28,15 @@ struct DpBuckets {
     const int* mw[3];
     int nmw[3];
     int* failflag;     // set by a W-wave or grid fill whose row wait gave up
-    // pairs filled by the device-wide strip pipeline (k_dp_grid)
+    // pairs whose strips are spread over one-wave workgroups (dp_grid_items)
     const int* grid;
     int ngrid;
     const int* gstrip0;                     // [ngrid + 1] first strip item of each pair
-    int* gnext;                             // the item counter
+    int* gnext;                             // the item counter, then [ngrid] strips done
     float* grows;                           // per pair nstrips x Lr floats at growoff[k]
     const unsigned long long* growoff;
     size_t growtot;                         // floats of all grid pairs' rows
-    int gworkers;                           // one-wave workgroups of the fill
+    int gworkers;                           // one-wave workgroups that take strips
     // any pair outside the one-wave list
     bool any_big() const { return nmw[0] > 0 || nmw[1] > 0 || nmw[2] > 0 || ngrid > 0; }
 };
