@@ -547,8 +547,11 @@ __device__ __forceinline__ void gapless_epilogue(const DevState& S, int p, const
     }
 }
 
+// Bound by VALU issue with 29 of 64 lanes live, so more waves fill the gaps: the
+// FP32 form is held to 96 VGPRs (of 102), 5 waves a SIMD (16 x 12,000 pairs: 4
+// waves 31.1 ms, 5 28.0, 6 30.0, 8 51; 1 x 25,000: 6.6, 6.0, 6.5, 10.8).
 template <int P>
-__global__ __launch_bounds__(RTHREADS) void k_refine_gapless(DevChunk Q, DevChunk R, DevState S, Geom G,
+__global__ __launch_bounds__(RTHREADS) __attribute__((amdgpu_waves_per_eu(P == 0 ? 5 : 1))) void k_refine_gapless(DevChunk Q, DevChunk R, DevState S, Geom G,
                                                               int dinv_on, const int* plist, SlotBest* parts) {
     __shared__ SlotBest lds[NGROUPS];
     __shared__ float tbest[NGROUPS][12];
