@@ -140,11 +140,10 @@ class GtaBatch:
         if self._q is None or self._r is None:
             self._check(lib().gta_process(self._h, C.byref(res)))
             return BlockResults(res)
-        # straight into the arrays handed out; the alignment section is mostly
-        # zeros, and its zero pages are never touched
+        # straight into the arrays handed out
         nq, nr = self._q.nstrs, self._r.nstrs
         arrays = (np.empty((nq, nr, GTA_ALN_NFIELDS), np.float32), np.empty((nq, nr, GTA_TFM_NFIELDS), np.float32),
-                  np.zeros(alignment_section_size(nq, self._q.nposs, nr, self._r.nposs), np.uint8))
+                  np.empty(alignment_section_size(nq, self._q.nposs, nr, self._r.nposs), np.uint8))
         self._check(lib().gta_process_into(self._h, nq * nr, *(a.ctypes.data for a in arrays), arrays[2].size,
                                            C.byref(res)))
         return BlockResults(res, arrays)

@@ -169,9 +169,10 @@ int gta_process(gta_ctx* ctx, gta_results* out);
 
 /* gta_process with the results in the caller's buffers: alndata for
  * pairs >= nq*nr records of 15 floats, tfms for as many transforms of 12, alns
- * at least gta_alignment_section_size() bytes, all zero on entry (fresh zero
- * pages cost nothing: only the rows of aligned pairs are written where they
- * are a small part of the section).  out's pointers are the caller's. */
+ * at least gta_alignment_section_size() bytes.  The buffers may hold anything
+ * on entry: every byte of the three sections is written (a section above 1 MiB
+ * is cleared by a thread of the call while the stage runs on the device).  On
+ * an error their contents are undefined.  out's pointers are the caller's. */
 int gta_process_into(gta_ctx* ctx, size_t pairs, float* alndata, float* tfms, char* alns, size_t alns_bytes,
                      gta_results* out);
 
