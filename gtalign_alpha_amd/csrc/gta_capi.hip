@@ -827,28 +827,14 @@ static int prepare_state(gta_ctx* c, DevState& S, size_t& alnsize) {
     return GTA_OK;
 }
 
-// Waves per workgroup of the DPRefine launches.  A launch ends with its longest
-// alignments, whose slots (about 6 per 40 positions) wait for each other in
-// the workgroup's 8 slot groups a wave, so larger workgroups make it shorter
-// until the device is full of them; then smaller ones leave fewer lanes idle
-// while a pair's last slots run.  28 launches with 1, 2 and 4 waves: 1 x 256
-// pairs 9.8, 6.4, 4.9 ms; 4 x 1,500 26.8, 16.4, 13.2; 4 x 2,500 85.7, 40.4, 27.1
-// (33 launches); 8 x 1,500 85.7, 41.4, 39.7; 1 x 25,000 64, 44.6, 47.0; 16 x
-// 12,000 202, 205, 258 (8 waves: 5.1, 18.7, 39, 62, 78, 455).  One-wave
-// workgroups also stage only alignments of up to rlds_cap32(1) positions in
-// LDS; longer ones are read from L2 in every pass.  An alignment is at most
-// min(Lq, Lr) long, so one wave is used when at most 15% of the pairs can have
-// longer ones (16 x 50,000: 7%, 0.85 s with two waves, 0.79 with one; 1 x
-// 500,000: 27%, 0.40 and 0.50).
-static int dprefine_waves(const gta_ctx* c) {
-    const double np = (double)c->q.len.size() * (double)c->r.len.size();
-    if (np <= 64.0 * c->ncu) return 4;
-    if (np <= 1024.0 * c->ncu) return 2;
+// whether at most 15% of the chunks' pairs can have alignments that one-wave
+// workgroups do not stage in LDS
+static bool fits_one_wave(const gta_ctx* c) {
     const int cap = rlds_cap32(1);
     long long ql = 0, rl = 0;
     for (int v : c->q.len) ql += v > cap;
     for (int v : c->r.len) rl += v > cap;
-    return (double)ql * (double)rl <= 0.15 * np ? 1 : 2;
+    return (double)ql * (double)rl <= 0.15 * (double)c->q.len.size() * (double)c->r.len.size();
 }
 
 static int run_stage(gta_ctx* c, double* seconds, double* cells) {
@@ -897,9 +883,8 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
         HIPCHK(c, (expr));                   \
         HIPCHK(c, ev_end());                 \
     } while (0)
-    int maxaln = std::min(c->q.len.front(), c->r.len.front());
-    const int dpr_waves = dprefine_waves(c);
-    RefineLaunch RL{dinv, 0, 0, 0, 0.f, std::min(maxaln, 1536), 0};
+    const int maxaln = std::min(c->q.len.front(), c->r.len.front());
+    const bool fits1 = fits_one_wave(c);
     // After each filter (the stage-1 prescreen, the -s threshold) the live
     // pairs are listed on the device.  The batched form's launches that follow
     // are persistent grids draining those lists (no host round trip: the
@@ -937,12 +922,9 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
         return launch_dp(Q, R, S, L, dpb, queue(lista, ltot), pgrid_dp, st);
     };
     auto refine = [&](int mode, int epi, int dpi, int maxdpi, float prescore) -> hipError_t {
-        RefineLaunch L = RL;
-        L.epi = epi; L.dpi = dpi; L.maxndpiters = maxdpi; L.prescore = prescore;
-        L.waves = mode == RM_DPREFINE_L ? dpr_waves : FINAL_WAVES;
-        // a persistent grid keeps 16 waves per CU whatever the workgroup size
-        const int pg = c->ncu * 16 / L.waves;
-        return launch_refine_dp(prec, mode, Q, R, S, G, L, rsp, queue(listb, ltot + 1), pg, st);
+        const RefineLaunch L{dinv, epi, dpi, maxdpi, prescore,
+                             refine_shape(prec, mode, c->ncu, (long long)np, maxaln, fits1)};
+        return launch_refine_dp(prec, mode, Q, R, S, G, L, rsp, queue(listb, ltot + 1), st);
     };
     // DPRefine<GAP0,PRESCREEN> (MpStage1.cpp:455-510)
     auto dprefine = [&](int gap0, float prescore, int maxdpi) -> int {
@@ -1173,6 +1155,13 @@ int gta_test_dp_score(gta_ctx* c, const float* tfms, const int* slotflags, int n
                               c->s_scout.as<float>(), st));
     HIPCHK(c, hipStreamSynchronize(st));
     HIPCHK(c, hipMemcpy(scores, c->s_scout.p, n * 4, hipMemcpyDeviceToHost));
+    return GTA_OK;
+}
+
+int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int* out) {
+    if (mode < RM_DPREFINE_L || mode > RM_PROD2L_L || ncu < 1 || pairs < 1 || maxaln < 1 || !out) return GTA_ERR_ARG;
+    const RefineShape s = refine_shape(prec != 0, mode, ncu, pairs, maxaln, fits1 != 0);
+    out[0] = s.waves; out[1] = s.wgs; out[2] = s.ldscap;
     return GTA_OK;
 }
 

@@ -2654,13 +2654,11 @@ hipError_t launch_dp_score(const DevChunk& Q, const DevChunk& R, const DevState&
 }
 hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChunk& R, const DevState& S,
                             const Geom& G, const RefineLaunch& L, const RefSplit& Sp, const WorkQ& wq,
-                            int pgrid, hipStream_t st) {
+                            hipStream_t st) {
     RefineParams prm{L.dinv, L.epi, L.dpi, L.maxndpiters, L.prescore};
-    // waves per workgroup of the unsplit pairs (the log search keeps RWAVES)
-    const int W = mode == RM_PROD2L ? RWAVES : L.waves;
-    const int ldscap = mode == RM_DPREFINE ? std::min(L.ldscap, rlds_cap32(W)) : L.ldscap;
+    const int W = L.shape.waves, ldscap = L.shape.ldscap;
     const size_t lds = (size_t)ldscap * 6 * sizeof(float);
-    const int nsmall = wq.items ? pgrid : (Sp.small ? Sp.nsmall : S.nq * S.nr);
+    const int nsmall = wq.items ? L.shape.wgs : (Sp.small ? Sp.nsmall : S.nq * S.nr);
     const bool phase2 = (mode == RM_FIN2 || mode == RM_PROD2);
     const bool full2 = (mode == RM_FIN2F || mode == RM_PROD2F);
     const int np = Sp.nbig > 0 ? nparts_for(phase2 ? G.maxnfragfcts

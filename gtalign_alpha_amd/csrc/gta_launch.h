@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include "gta_device.h"
 
 namespace gta {
@@ -55,12 +56,51 @@ struct RefSplit {
     void* partbuf;
 };
 
+// Workgroups of a refinement launch over the DP alignments.
+struct RefineShape {
+    int waves;         // per workgroup of unsplit pairs
+    int wgs;           // workgroups of a persistent grid: 16 waves per CU
+    int ldscap;        // alignments up to this length are staged in LDS
+};
+
+// Waves per workgroup of the DPRefine launches over a chunk of `pairs` pairs.
+// A launch ends with its longest alignments, whose slots (about 6 per 40
+// positions) wait for each other in the workgroup's 8 slot groups a wave, so
+// larger workgroups make it shorter until the device is full of them; then
+// smaller ones leave fewer lanes idle while a pair's last slots run.  28
+// launches with 1, 2 and 4 waves: 1 x 256 pairs 9.8, 6.4, 4.9 ms; 4 x 1,500
+// 26.8, 16.4, 13.2; 4 x 2,500 85.7, 40.4, 27.1 (33 launches); 8 x 1,500 85.7,
+// 41.4, 39.7; 1 x 25,000 64, 44.6, 47.0; 16 x 12,000 202, 205, 258 (8 waves:
+// 5.1, 18.7, 39, 62, 78, 455).  One-wave workgroups also stage only alignments
+// of up to rlds_cap32(1) positions in LDS; longer ones are read from L2 in
+// every pass.  An alignment is at most min(Lq, Lr) long, so one wave is used
+// when at most 15% of the pairs can have longer ones (fits1; 16 x 50,000: 7%,
+// 0.85 s with two waves, 0.79 with one; 1 x 500,000: 27%, 0.40 and 0.50).
+inline int dprefine_waves(int ncu, long long pairs, bool fits1) {
+    if (pairs <= 64ll * ncu) return 4;
+    return pairs <= 1024ll * ncu || !fits1 ? 2 : 1;
+}
+
+// The shape of the launch of refinement `mode` over `pairs` pairs of alignments
+// of up to `maxaln` positions.  The log search's steps run in order in one slot
+// group, so its pairs take workgroups of REFINE_WAVES, the other final modes'
+// workgroups of FINAL_WAVES.  The FP32 forms stage in LDS what leaves room for
+// 16 waves per CU; the FP64 ones, which run 8, up to 1,536 positions.
+inline RefineShape refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, bool fits1) {
+    RefineShape s;
+    s.waves = mode == RM_DPREFINE_L ? dprefine_waves(ncu, pairs, fits1)
+              : mode == RM_PROD2L_L ? REFINE_WAVES : FINAL_WAVES;
+    s.wgs = ncu * 16 / s.waves;
+    s.ldscap = std::min(maxaln, 1536);
+    if (prec == 0 || mode == RM_DPREFINE_L) s.ldscap = std::min(s.ldscap, rlds_cap32(s.waves));
+    return s;
+}
+
 struct RefineLaunch {
     int dinv;
     int epi, dpi, maxndpiters;
     float prescore;
-    int ldscap;        // alignments up to this length are staged in LDS
-    int waves;         // waves per workgroup of unsplit pairs: DPRefine 1, 2 or 4, the others FINAL_WAVES
+    RefineShape shape;
 };
 
 hipError_t launch_secstr(const DevChunk& C, hipStream_t st);
@@ -93,7 +133,7 @@ hipError_t launch_dp_score(const DevChunk& Q, const DevChunk& R, const DevState&
 // FIN2, PROD1, PROD2); DPREFINE is a search and stays FP32
 hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChunk& R,
                             const DevState& S, const Geom& G, const RefineLaunch& L, const RefSplit& Sp,
-                            const WorkQ& wq, int pgrid, hipStream_t st);
+                            const WorkQ& wq, hipStream_t st);
 // bytes of one part record (partbuf entries)
 size_t part_record_bytes();
 hipError_t launch_prod_aln(const DevChunk& Q, const DevChunk& R, const DevState& S, char* alns,

@@ -1,0 +1,57 @@
+"""The workgroups of the refinement launches (host rule, no device), and the
+batched form of the log search with more pairs than its persistent grid has
+workgroups."""
+import numpy as np
+import pytest
+
+from gtalign_alpha_amd import synth
+from gtalign_alpha_amd.batch import GtaBatch, lib
+from gtalign_alpha_amd.capi import PREC_FP32, PREC_MIXED, REF_LOG, default_options
+from gtalign_alpha_amd.chunk import Chunk
+
+NCU = 256
+DPREFINE, LOG = 0, 7
+
+
+def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1, n=3):
+    out = np.zeros(n, np.int32)
+    assert lib().gta_test_refine_shape(prec, mode, NCU, pairs, maxaln, fits1, out.ctypes.data) == 0
+    return out.tolist()
+
+
+@pytest.mark.parametrize("prec", [PREC_FP32, PREC_MIXED])
+@pytest.mark.parametrize("mode", range(8))
+@pytest.mark.parametrize("pairs", [1, 1000, 100000, 1000000])
+def test_persistent_grid_fills_the_device(prec, mode, pairs):
+    """16 waves per CU whatever the workgroup size, and in the FP32 forms LDS
+    (2 KB a wave and the staged alignment) for all of them."""
+    waves, wgs, cap = shape(prec, mode, pairs)
+    assert waves * wgs == 16 * NCU
+    assert mode != LOG or waves == 2            # its steps run in one slot group
+    if prec == PREC_FP32 or mode == DPREFINE:
+        assert wgs // NCU * (2048 * waves + 24 * cap) <= 160 * 1024
+    assert shape(prec, mode, pairs, maxaln=100)[2] == 100
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [PREC_FP32, PREC_MIXED], ids=["fp32", "mixed"])
+def test_batched_log_search(prec):
+    """2,500 copies of one chain: every pair reaches the log search, which has
+    8 workgroups per CU."""
+    rng = np.random.default_rng(6)
+    x = synth.chain(31, 44)
+    rs = [synth.rigid_copy(rng, x, 0.1 + 0.1 * (i % 9)) for i in range(2500)]
+    q, r = Chunk.from_structures([x], ["A" * 44]), Chunk.from_structures(rs, ["A" * 44] * 2500)
+    got = []
+    for batched in (0, 1):
+        with GtaBatch(0, default_options(refinement=REF_LOG, precision=prec, batched=batched), max_qrys=1,
+                      max_qry_poss=q.nposs, max_refs=r.nstrs, max_ref_poss=r.nposs) as b:
+            b.TransferQueryPMDataToDevice(q)
+            b.TransferCPMDataToDevice(r)
+            got.append([b.ProcessBlock() for _ in range(3 if batched else 1)])
+    want = got[0][0]
+    assert (want.alndata[..., 4] > 0).sum() > 8 * NCU
+    for g in got[1]:
+        assert np.array_equal(g.alndata, want.alndata)
+        assert np.array_equal(g.tfms, want.tfms)
+        assert np.array_equal(g.alns, want.alns)
