@@ -1161,7 +1161,7 @@ int gta_test_dp_score(gta_ctx* c, const float* tfms, const int* slotflags, int n
 int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int* out) {
     if (mode < RM_DPREFINE_L || mode > RM_PROD2L_L || ncu < 1 || pairs < 1 || maxaln < 1 || !out) return GTA_ERR_ARG;
     const RefineShape s = refine_shape(prec != 0, mode, ncu, pairs, maxaln, fits1 != 0);
-    out[0] = s.waves; out[1] = s.wgs; out[2] = s.ldscap;
+    out[0] = s.waves; out[1] = s.wgs; out[2] = s.ldscap; out[3] = s.split_waves; out[4] = s.split_ldscap;
     return GTA_OK;
 }
 

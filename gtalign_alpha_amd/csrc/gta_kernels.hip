@@ -2656,8 +2656,8 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
                             const Geom& G, const RefineLaunch& L, const RefSplit& Sp, const WorkQ& wq,
                             hipStream_t st) {
     RefineParams prm{L.dinv, L.epi, L.dpi, L.maxndpiters, L.prescore};
-    const int W = L.shape.waves, ldscap = L.shape.ldscap;
-    const size_t lds = (size_t)ldscap * 6 * sizeof(float);
+    const int W = L.shape.waves, ldscap = L.shape.ldscap, sldscap = L.shape.split_ldscap;
+    const size_t lds = (size_t)ldscap * 6 * sizeof(float), slds = (size_t)sldscap * 6 * sizeof(float);
     const int nsmall = wq.items ? L.shape.wgs : (Sp.small ? Sp.nsmall : S.nq * S.nr);
     const bool phase2 = (mode == RM_FIN2 || mode == RM_PROD2);
     const bool full2 = (mode == RM_FIN2F || mode == RM_PROD2F);
@@ -2674,8 +2674,8 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
             hipLaunchKernelGGL((k_refine_dp<PP, MM, W>), dim3(nsmall), dim3(W * GTA_WAVE), lds, st, Q, R, S, G, prm, \
                                ldscap, Sp.small, (SlotBest*)nullptr, wq);                                    \
         if (Sp.nbig > 0) {                                                                                     \
-            hipLaunchKernelGGL((k_refine_dp<PP, MM, WB>), dim3(Sp.nbig, np), dim3(WB * GTA_WAVE), lds, st, Q, R, S, \
-                               G, prm, ldscap, Sp.big, parts, WorkQ{});                                      \
+            hipLaunchKernelGGL((k_refine_dp<PP, MM, WB>), dim3(Sp.nbig, np), dim3(WB * GTA_WAVE), slds, st, Q, R, S, \
+                               G, prm, sldscap, Sp.big, parts, WorkQ{});                                     \
             hipLaunchKernelGGL((k_merge_parts<2, MM>), dim3((Sp.nbig + 63) / 64), dim3(64), 0, st, Q, R, S,   \
                                prm, Sp.big, Sp.nbig, np, parts);                                               \
         }                                                                                                      \
@@ -2689,8 +2689,8 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
             hipLaunchKernelGGL((k_refine_dp<PP, RM_PROD2L>), dim3(nsmall), dim3(RTHREADS), lds, st, Q, R, S, G, \
                                prm, ldscap, Sp.small, (SlotBest*)nullptr, wq);                               \
         if (Sp.nbig > 0)                                                                                       \
-            hipLaunchKernelGGL((k_refine_dp<PP, RM_PROD2L>), dim3(Sp.nbig), dim3(RTHREADS), lds, st, Q, R, S, G,\
-                               prm, ldscap, Sp.big, (SlotBest*)nullptr, WorkQ{});                            \
+            hipLaunchKernelGGL((k_refine_dp<PP, RM_PROD2L>), dim3(Sp.nbig), dim3(RTHREADS), slds, st, Q, R, S, G,\
+                               prm, sldscap, Sp.big, (SlotBest*)nullptr, WorkQ{});                           \
     } while (0)
 #define GTA_RLM(PP)                                      \
     switch (mode) {                                      \

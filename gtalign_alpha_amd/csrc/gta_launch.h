@@ -61,6 +61,8 @@ struct RefineShape {
     int waves;         // per workgroup of unsplit pairs
     int wgs;           // workgroups of a persistent grid: 16 waves per CU
     int ldscap;        // alignments up to this length are staged in LDS
+    int split_waves;   // the same of split pairs' workgroups
+    int split_ldscap;
 };
 
 // Waves per workgroup of the DPRefine launches over a chunk of `pairs` pairs.
@@ -84,15 +86,22 @@ inline int dprefine_waves(int ncu, long long pairs, bool fits1) {
 // The shape of the launch of refinement `mode` over `pairs` pairs of alignments
 // of up to `maxaln` positions.  The log search's steps run in order in one slot
 // group, so its pairs take workgroups of REFINE_WAVES, the other final modes'
-// workgroups of FINAL_WAVES.  The FP32 forms stage in LDS what leaves room for
-// 16 waves per CU; the FP64 ones, which run 8, up to 1,536 positions.
+// workgroups of FINAL_WAVES; split pairs, each many workgroups, take at most
+// REFINE_WAVES.  The FP32 forms stage in LDS what leaves room for 16 waves per
+// CU at their own workgroup size (1 x 200 pairs of 2,900 residues, split: with
+// the unsplit pairs' LDS 102 ms of DPRefine, with their own 68); the FP64 ones,
+// which run 8, up to 1,536 positions.
 inline RefineShape refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, bool fits1) {
     RefineShape s;
     s.waves = mode == RM_DPREFINE_L ? dprefine_waves(ncu, pairs, fits1)
               : mode == RM_PROD2L_L ? REFINE_WAVES : FINAL_WAVES;
     s.wgs = ncu * 16 / s.waves;
-    s.ldscap = std::min(maxaln, 1536);
-    if (prec == 0 || mode == RM_DPREFINE_L) s.ldscap = std::min(s.ldscap, rlds_cap32(s.waves));
+    s.split_waves = std::min(s.waves, REFINE_WAVES);
+    s.ldscap = s.split_ldscap = std::min(maxaln, 1536);
+    if (prec == 0 || mode == RM_DPREFINE_L) {
+        s.ldscap = std::min(s.ldscap, rlds_cap32(s.waves));
+        s.split_ldscap = std::min(s.split_ldscap, rlds_cap32(s.split_waves));
+    }
     return s;
 }
 

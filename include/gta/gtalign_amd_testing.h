@@ -75,7 +75,8 @@ int gta_test_set_split(gta_ctx* ctx, int min_len, int seeds_per_part, int slots_
  * most maxaln positions; fits1: few of them exceed what one wave's workgroups
  * stage in LDS.  out[0] receives the waves per workgroup, out[1] the workgroups
  * of a persistent grid, out[2] the longest alignment staged in LDS (24 bytes a
- * position). */
+ * position), out[3] and out[4] the waves and the staged length of the split
+ * pairs' workgroups. */
 int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int* out);
 
 /* The pair score d0^2 / (d0^2 + d^2) of the DP cells and TM-score passes

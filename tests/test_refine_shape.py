@@ -13,8 +13,8 @@ NCU = 256
 DPREFINE, LOG = 0, 7
 
 
-def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1, n=3):
-    out = np.zeros(n, np.int32)
+def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1):
+    out = np.zeros(5, np.int32)
     assert lib().gta_test_refine_shape(prec, mode, NCU, pairs, maxaln, fits1, out.ctypes.data) == 0
     return out.tolist()
 
@@ -25,12 +25,20 @@ def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1, n=3):
 def test_persistent_grid_fills_the_device(prec, mode, pairs):
     """16 waves per CU whatever the workgroup size, and in the FP32 forms LDS
     (2 KB a wave and the staged alignment) for all of them."""
-    waves, wgs, cap = shape(prec, mode, pairs)
+    waves, wgs, cap, _, _ = shape(prec, mode, pairs)
     assert waves * wgs == 16 * NCU
     assert mode != LOG or waves == 2            # its steps run in one slot group
     if prec == PREC_FP32 or mode == DPREFINE:
         assert wgs // NCU * (2048 * waves + 24 * cap) <= 160 * 1024
     assert shape(prec, mode, pairs, maxaln=100)[2] == 100
+
+
+@pytest.mark.parametrize("mode", range(8))
+@pytest.mark.parametrize("pairs", [1, 1000, 100000, 1000000])
+def test_split_workgroups_leave_room_for_16_waves(mode, pairs):
+    """The LDS of a split pair's workgroups follows from their own waves."""
+    _, _, _, waves, cap = shape(PREC_FP32, mode, pairs)
+    assert waves <= 2 and 16 // waves * (2048 * waves + 24 * cap) <= 160 * 1024
 
 
 @pytest.mark.gpu
