@@ -82,7 +82,7 @@ def lib():
         L.gta_test_set_dp_grid.restype = C.c_int
         L.gta_test_set_split.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int]
         L.gta_test_set_split.restype = C.c_int
-        L.gta_test_refine_shape.argtypes = [C.c_int] * 3 + [C.c_longlong] + [C.c_int] * 2 + [C.c_void_p]
+        L.gta_test_refine_shape.argtypes = [C.c_int] * 3 + [C.c_longlong] + [C.c_int] * 3 + [C.c_void_p]
         L.gta_test_refine_shape.restype = C.c_int
         L.gta_test_pair_score.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         L.gta_test_pair_score.restype = C.c_int

@@ -65,22 +65,37 @@ struct RefineShape {
     int split_ldscap;
 };
 
-// Waves per workgroup of the DPRefine launches over a chunk of `pairs` pairs.
-// A launch ends with its longest alignments, whose slots (about 6 per 40
-// positions) wait for each other in the workgroup's 8 slot groups a wave, so
-// larger workgroups make it shorter until the device is full of them; then
-// smaller ones leave fewer lanes idle while a pair's last slots run.  28
-// launches with 1, 2 and 4 waves: 1 x 256 pairs 9.8, 6.4, 4.9 ms; 4 x 1,500
-// 26.8, 16.4, 13.2; 4 x 2,500 85.7, 40.4, 27.1 (33 launches); 8 x 1,500 85.7,
-// 41.4, 39.7; 1 x 25,000 64, 44.6, 47.0; 16 x 12,000 202, 205, 258 (8 waves:
-// 5.1, 18.7, 39, 62, 78, 455).  One-wave workgroups also stage only alignments
-// of up to rlds_cap32(1) positions in LDS; longer ones are read from L2 in
-// every pass.  An alignment is at most min(Lq, Lr) long, so one wave is used
-// when at most 15% of the pairs can have longer ones (fits1; 16 x 50,000: 7%,
-// 0.85 s with two waves, 0.79 with one; 1 x 500,000: 27%, 0.40 and 0.50).
-inline int dprefine_waves(int ncu, long long pairs, bool fits1) {
-    if (pairs <= 64ll * ncu) return 4;
-    return pairs <= 1024ll * ncu || !fits1 ? 2 : 1;
+// Waves per workgroup of the DPRefine launches over a chunk of `pairs` pairs
+// whose alignments have up to `maxaln` positions.  A launch ends with its longest
+// alignments, whose slots (about 6 per 40 positions) wait for each other in the
+// workgroup's 8 slot groups a wave, so larger workgroups make it shorter until
+// the device is full of them; then smaller ones leave fewer lanes idle while a
+// pair's last slots run.  The longer the longest alignment is beside the others,
+// the more pairs it takes to hide it: the lines follow maxaln.  28 launches with
+// 1, 2 and 4 waves, ms:
+//   up to 90 positions: 1,000 pairs 3.0, 2.0, 2.0; 4,500 2.9, 2.6, 2.9; 10,000 3.9,
+//     3.7, 4.2; 16,000 4.6, 4.7, 5.7; 64,000 9.2, 14.1, 22.3
+//   up to 140: 12,800 pairs 13.3, 11.1, 12.5; 44,000 27.3, 27.9, 38.0
+//   up to 200: 4,000 pairs 12.2, 7.7, 6.1; 16,000 14.4, 13.2, 18.0; 40,000 20.5,
+//     22.1, 34.7; 64,000 37, 44, 71
+//   up to 300: 15,000 pairs 18.1, 12.4, 12.1; 54,000 45.6, 43.9, 53.6; 79,000
+//     45.0, 49.9, 80.8
+//   up to 1,000: 4 x 1,500 24.7, 15.1, 11.3; 16,000 pairs 128, 56, 43; 64,000 153,
+//     128, 156; 16 x 12,000 176, 174, 216; 16 x 50,000 661, 712, 888
+// One-wave workgroups also stage only alignments of up to rlds_cap32(1)
+// positions in LDS; longer ones are read from L2 in every pass, so one wave is
+// used when at most 15% of the pairs can have longer ones (fits1; 16 x 50,000: 7%;
+// 1 x 500,000: 27%, 0.40 s with two waves and 0.50 with one).
+// The at most 8 slots of up to 47 positions fit one wave: 99 pairs 0.69, 0.74,
+// 0.76; 16,000 2.1, 2.8, 3.2; 64,000 5.4, 9.3, 11.8.  In a small batched chunk the
+// 4,096 one-wave workgroups of the persistent grid would take longer to find
+// the queue empty: 54 pairs 2.5, 2.0, 1.8; 10,000 3.7, 3.4, 3.1; 30,000 8.0, 8.7,
+// 8.4.
+inline int dprefine_waves(int ncu, long long pairs, int maxaln, bool fits1, bool batched) {
+    const double percu = (double)pairs / ncu;
+    if (maxaln <= 47) return batched && percu <= 64.0 ? 4 : 1;
+    if (percu <= std::min(64.0, 4.0 + maxaln / 5.0)) return 4;
+    return percu <= std::min(1024.0, 0.9 * maxaln) || !fits1 ? 2 : 1;
 }
 
 // The shape of the launch of refinement `mode` over `pairs` pairs of alignments
@@ -91,9 +106,10 @@ inline int dprefine_waves(int ncu, long long pairs, bool fits1) {
 // CU at their own workgroup size (1 x 200 pairs of 2,900 residues, split: with
 // the unsplit pairs' LDS 102 ms of DPRefine, with their own 68); the FP64 ones,
 // which run 8, up to 1,536 positions.
-inline RefineShape refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, bool fits1) {
+inline RefineShape refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, bool fits1,
+                                bool batched) {
     RefineShape s;
-    s.waves = mode == RM_DPREFINE_L ? dprefine_waves(ncu, pairs, fits1)
+    s.waves = mode == RM_DPREFINE_L ? dprefine_waves(ncu, pairs, maxaln, fits1, batched)
               : mode == RM_PROD2L_L ? REFINE_WAVES : FINAL_WAVES;
     s.wgs = ncu * 16 / s.waves;
     s.split_waves = std::min(s.waves, REFINE_WAVES);

@@ -73,11 +73,12 @@ int gta_test_set_split(gta_ctx* ctx, int min_len, int seeds_per_part, int slots_
  * precision prec (0 FP32, 1 mixed), mode 0 DPRefine, 1-6 the final stage's
  * modes, 7 the log search; ncu compute units, `pairs` pairs, alignments of at
  * most maxaln positions; fits1: few of them exceed what one wave's workgroups
- * stage in LDS.  out[0] receives the waves per workgroup, out[1] the workgroups
+ * stage in LDS; batched: the batched form.  out[0] receives the waves per workgroup, out[1] the workgroups
  * of a persistent grid, out[2] the longest alignment staged in LDS (24 bytes a
  * position), out[3] and out[4] the waves and the staged length of the split
  * pairs' workgroups. */
-int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int* out);
+int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int batched,
+                          int* out);
 
 /* The pair score d0^2 / (d0^2 + d^2) of the DP cells and TM-score passes
  * (scoringbase.h:61-65) for n caller-given operand pairs: out[i] receives

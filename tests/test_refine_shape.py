@@ -1,6 +1,5 @@
 """The workgroups of the refinement launches (host rule, no device), and the
-batched form of the log search with more pairs than its persistent grid has
-workgroups."""
+batched form with more pairs than a persistent grid has workgroups."""
 import numpy as np
 import pytest
 
@@ -13,9 +12,9 @@ NCU = 256
 DPREFINE, LOG = 0, 7
 
 
-def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1):
+def shape(prec, mode, pairs=1000, maxaln=4000, fits1=1, batched=0):
     out = np.zeros(5, np.int32)
-    assert lib().gta_test_refine_shape(prec, mode, NCU, pairs, maxaln, fits1, out.ctypes.data) == 0
+    assert lib().gta_test_refine_shape(prec, mode, NCU, pairs, maxaln, fits1, batched, out.ctypes.data) == 0
     return out.tolist()
 
 
@@ -31,6 +30,19 @@ def test_persistent_grid_fills_the_device(prec, mode, pairs):
     if prec == PREC_FP32 or mode == DPREFINE:
         assert wgs // NCU * (2048 * waves + 24 * cap) <= 160 * 1024
     assert shape(prec, mode, pairs, maxaln=100)[2] == 100
+
+
+@pytest.mark.parametrize("maxaln,pairs,waves", [
+    (47, 256, 1), (47, 64000, 1), (90, 4000, 4), (90, 16000, 2), (90, 64000, 1), (150, 16000, 2), (200, 8000, 4),
+    (200, 16000, 2), (200, 64000, 1), (300, 15000, 4), (300, 80000, 1), (1000, 16384, 4), (1000, 16385, 2),
+    (1000, 100000, 2), (1000, 800000, 1), (65535, 1, 4), (65535, 262144, 2), (65535, 262145, 1)])
+def test_dprefine_waves_follow_length_and_number(maxaln, pairs, waves):
+    """Chunks of short chains take small workgroups, however few their pairs."""
+    assert shape(PREC_FP32, DPREFINE, pairs, maxaln)[0] == waves
+    if waves == 1:                              # never where many alignments exceed its LDS
+        assert shape(PREC_FP32, DPREFINE, pairs, maxaln, fits1=0)[0] == (1 if maxaln <= 47 else 2)
+    small = maxaln <= 47 and pairs <= 64 * NCU  # a persistent grid of one-wave workgroups only for many pairs
+    assert shape(PREC_FP32, DPREFINE, pairs, maxaln, batched=1)[0] == (4 if small else waves)
 
 
 @pytest.mark.parametrize("mode", range(8))
@@ -50,16 +62,35 @@ def test_batched_log_search(prec):
     x = synth.chain(31, 44)
     rs = [synth.rigid_copy(rng, x, 0.1 + 0.1 * (i % 9)) for i in range(2500)]
     q, r = Chunk.from_structures([x], ["A" * 44]), Chunk.from_structures(rs, ["A" * 44] * 2500)
+    want = batched_equals_plain(q, r, refinement=REF_LOG, precision=prec)
+    assert (want.alndata[..., 4] > 0).sum() > 8 * NCU
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nr,hi,waves", [(1000, 170, 4), (2500, 170, 2), (2500, 60, 1)])
+def test_batched_dprefine_of_unchanged_alignments(nr, hi, waves):
+    """Persistent workgroups of each size that take several pairs, many of
+    whose refinements end at once because their alignment did not change."""
+    rng = np.random.default_rng(8)
+    seeds = [synth.chain(300 + i, int(rng.integers(30, hi + 1))) for i in range(7)] + [synth.chain(299, hi)]
+    rs = [synth.rigid_copy(rng, seeds[i % 8], 0.2 + 0.4 * (i % 7)) for i in range(nr)]
+    q, r = (Chunk.from_structures(xs, [synth.residues(rng, len(x)) for x in xs]) for xs in (seeds, rs))
+    assert shape(PREC_FP32, DPREFINE, 8 * nr, hi, batched=1)[0] == waves
+    batched_equals_plain(q, r, prescore=0.0)
+
+
+def batched_equals_plain(q, r, **kw):
+    """The batched form's first call and two replays equal the plain form's bits."""
     got = []
     for batched in (0, 1):
-        with GtaBatch(0, default_options(refinement=REF_LOG, precision=prec, batched=batched), max_qrys=1,
-                      max_qry_poss=q.nposs, max_refs=r.nstrs, max_ref_poss=r.nposs) as b:
+        with GtaBatch(0, default_options(batched=batched, **kw), max_qrys=q.nstrs, max_qry_poss=q.nposs,
+                      max_refs=r.nstrs, max_ref_poss=r.nposs) as b:
             b.TransferQueryPMDataToDevice(q)
             b.TransferCPMDataToDevice(r)
             got.append([b.ProcessBlock() for _ in range(3 if batched else 1)])
     want = got[0][0]
-    assert (want.alndata[..., 4] > 0).sum() > 8 * NCU
     for g in got[1]:
         assert np.array_equal(g.alndata, want.alndata)
         assert np.array_equal(g.tfms, want.tfms)
         assert np.array_equal(g.alns, want.alns)
+    return want
