@@ -922,8 +922,10 @@ static int run_stage(gta_ctx* c, double* seconds, double* cells) {
         return launch_dp(Q, R, S, L, dpb, queue(lista, ltot), pgrid_dp, st);
     };
     auto refine = [&](int mode, int epi, int dpi, int maxdpi, float prescore) -> hipError_t {
+        // DPRefine's workgroups follow the chunk, the final stage's the pairs left
+        const long long pairs = mode == RM_DPREFINE_L ? (long long)np : batched ? 0 : rsp.nsmall;
         const RefineLaunch L{dinv, epi, dpi, maxdpi, prescore,
-                             refine_shape(prec, mode, c->ncu, (long long)np, maxaln, fits1, batched)};
+                             refine_shape(prec, mode, c->ncu, pairs, maxaln, fits1, batched)};
         return launch_refine_dp(prec, mode, Q, R, S, G, L, rsp, queue(listb, ltot + 1), st);
     };
     // DPRefine<GAP0,PRESCREEN> (MpStage1.cpp:455-510)
@@ -1160,7 +1162,7 @@ int gta_test_dp_score(gta_ctx* c, const float* tfms, const int* slotflags, int n
 
 int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int batched,
                           int* out) {
-    if (mode < RM_DPREFINE_L || mode > RM_PROD2L_L || ncu < 1 || pairs < 1 || maxaln < 1 || !out) return GTA_ERR_ARG;
+    if (mode < RM_DPREFINE_L || mode > RM_PROD2L_L || ncu < 1 || pairs < 0 || maxaln < 1 || !out) return GTA_ERR_ARG;
     const RefineShape s = refine_shape(prec != 0, mode, ncu, pairs, maxaln, fits1 != 0, batched != 0);
     out[0] = s.waves; out[1] = s.wgs; out[2] = s.ldscap; out[3] = s.split_waves; out[4] = s.split_ldscap;
     return GTA_OK;

@@ -40,11 +40,7 @@ enum { CCM00 = 0, CVq0 = 9, CVr0 = 12, NALN = 15, NCC = 16 };
 // waiting for its last slots small and leave LDS to stage alignments of up to
 // 682 positions
 constexpr int REFINE_WAVES = 2;
-// and of the final stage's refinements, which few pairs reach and whose second
-// phases run 128 slots a pair: 64 slot groups take them in two rounds instead of
-// 8 (4 launches: 1 x 256 pairs 1.7 -> 0.6 ms, 4 x 1,500 3.1 -> 0.9, 8 x 1,500 in
-// mixed precision 6.4 -> 2.1, 16 x 12,000 5.0 -> 3.4; 1 x 900 equal chains 0.6 ->
-// 0.8)
+// and the most of the final stage's refinements (final_waves, gta_launch.h)
 constexpr int FINAL_WAVES = 8;
 // Alignments staged in LDS by the FP32 refinements (24 B per position) in
 // workgroups of W waves, 16 waves per CU: the workgroups' fixed LDS (just

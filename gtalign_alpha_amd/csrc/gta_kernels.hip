@@ -2681,7 +2681,11 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
         }                                                                                                      \
     } while (0)
     // the final stage's modes
-#define GTA_RL(PP, MM) GTA_RLW(PP, MM, FINAL_WAVES, RWAVES)
+#define GTA_RL(PP, MM)                                           \
+    do {                                                         \
+        if (W == FINAL_WAVES) GTA_RLW(PP, MM, FINAL_WAVES, RWAVES); \
+        else GTA_RLW(PP, MM, FINAL_WAVES / 2, RWAVES);           \
+    } while (0)
     // the log search's steps run in order within one workgroup: no split
 #define GTA_RL_LOG(PP)                                                                                         \
     do {                                                                                                       \
@@ -2701,9 +2705,9 @@ hipError_t launch_refine_dp(int prec, int mode, const DevChunk& Q, const DevChun
             break;                                       \
         case RM_FIN1: GTA_RL(PP, RM_FIN1); break;         \
         case RM_FIN2: GTA_RL(PP, RM_FIN2); break;         \
-        case RM_FIN2F: GTA_RL(PP, RM_FIN2F); break;       \
+        case RM_FIN2F: GTA_RLW(PP, RM_FIN2F, FINAL_WAVES, RWAVES); break;       \
         case RM_PROD1: GTA_RL(PP, RM_PROD1); break;       \
-        case RM_PROD2F: GTA_RL(PP, RM_PROD2F); break;     \
+        case RM_PROD2F: GTA_RLW(PP, RM_PROD2F, FINAL_WAVES, RWAVES); break;     \
         case RM_PROD2L: GTA_RL_LOG(PP); break;            \
         default: GTA_RL(PP, RM_PROD2); break;             \
     }

@@ -98,19 +98,40 @@ inline int dprefine_waves(int ncu, long long pairs, int maxaln, bool fits1, bool
     return percu <= std::min(1024.0, 0.9 * maxaln) || !fits1 ? 2 : 1;
 }
 
+// Waves per workgroup of the final stage's launches over `live` pairs (0: not
+// known, as in the batched form).  Few pairs reach it, whose second phases run
+// 128 slots: 64 slot groups take them in two rounds.  Where the pairs keep every
+// CU busy, half as many groups leave fewer of them idle and let a second
+// workgroup work while one waits; the longer the longest alignment, the later.
+// 4 launches with 8 and 4 waves, ms (longest alignment, pairs per CU):
+//   FP32: 211, 1.6 0.26, 0.24; 221, 4.0 0.90, 1.13; 334, 5.8 1.19, 1.48; 400, 5.9
+//     0.99, 1.10; 400, 11.7 1.67, 1.53; 546, 13 2.95, 2.75; 78, 6.7 0.56, 0.54; 100,
+//     15.6 1.30, 0.91
+//   FP64, of which a CU holds 8 waves: 100, 1.0 0.20, 0.20; 211, 3.5 0.77, 0.56;
+//     400, 2.3 0.84, 0.81; 400, 3.5 1.10, 0.96; 568, 4.1 2.03, 2.97; 900, 2.3 2.13, 2.50;
+//     221, 23 7.3, 5.3
+inline int final_waves(int prec, int ncu, long long live, int maxaln) {
+    const double percu = (double)live / ncu;
+    return percu <= (prec ? std::max(1.0, maxaln / 130.0) : std::max(2.0, maxaln / 50.0)) ? FINAL_WAVES
+                                                                                         : FINAL_WAVES / 2;
+}
+
 // The shape of the launch of refinement `mode` over `pairs` pairs of alignments
-// of up to `maxaln` positions.  The log search's steps run in order in one slot
-// group, so its pairs take workgroups of REFINE_WAVES, the other final modes'
-// workgroups of FINAL_WAVES; split pairs, each many workgroups, take at most
-// REFINE_WAVES.  The FP32 forms stage in LDS what leaves room for 16 waves per
-// CU at their own workgroup size (1 x 200 pairs of 2,900 residues, split: with
-// the unsplit pairs' LDS 102 ms of DPRefine, with their own 68); the FP64 ones,
-// which run 8, up to 1,536 positions.
+// of up to `maxaln` positions (the final stage's: the live pairs, 0 where the
+// host does not know them).  The log search's steps run in order in one slot
+// group, so its pairs take workgroups of REFINE_WAVES; the FULLA searches, of
+// 768 slots a pair, workgroups of FINAL_WAVES; split pairs, each many
+// workgroups, take at most REFINE_WAVES.  The FP32 forms stage in LDS what leaves
+// room for 16 waves per CU at their own workgroup size (1 x 200 pairs of 2,900
+// residues, split: with the unsplit pairs' LDS 102 ms of DPRefine, with their own
+// 68); the FP64 ones, which run 8, up to 1,536 positions.
 inline RefineShape refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, bool fits1,
                                 bool batched) {
     RefineShape s;
     s.waves = mode == RM_DPREFINE_L ? dprefine_waves(ncu, pairs, maxaln, fits1, batched)
-              : mode == RM_PROD2L_L ? REFINE_WAVES : FINAL_WAVES;
+              : mode == RM_PROD2L_L ? REFINE_WAVES
+              : mode == RM_FIN2F_L || mode == RM_PROD2F_L ? FINAL_WAVES
+                                                          : final_waves(prec, ncu, pairs, maxaln);
     s.wgs = ncu * 16 / s.waves;
     s.split_waves = std::min(s.waves, REFINE_WAVES);
     s.ldscap = s.split_ldscap = std::min(maxaln, 1536);

@@ -71,12 +71,13 @@ int gta_test_set_split(gta_ctx* ctx, int min_len, int seeds_per_part, int slots_
 
 /* The workgroups that the stage gives a refinement launch (no device needed):
  * precision prec (0 FP32, 1 mixed), mode 0 DPRefine, 1-6 the final stage's
- * modes, 7 the log search; ncu compute units, `pairs` pairs, alignments of at
- * most maxaln positions; fits1: few of them exceed what one wave's workgroups
- * stage in LDS; batched: the batched form.  out[0] receives the waves per workgroup, out[1] the workgroups
- * of a persistent grid, out[2] the longest alignment staged in LDS (24 bytes a
- * position), out[3] and out[4] the waves and the staged length of the split
- * pairs' workgroups. */
+ * modes, 7 the log search; ncu compute units, `pairs` pairs (in the final
+ * stage those left, 0: not known), alignments of at most maxaln positions;
+ * fits1: few of them exceed what one wave's workgroups stage in LDS; batched:
+ * the batched form.  out[0] receives the waves per workgroup, out[1] the
+ * workgroups of a persistent grid, out[2] the longest alignment staged in LDS
+ * (24 bytes a position), out[3] and out[4] the waves and the staged length of
+ * the split pairs' workgroups. */
 int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxaln, int fits1, int batched,
                           int* out);
 

@@ -45,6 +45,44 @@ def test_dprefine_waves_follow_length_and_number(maxaln, pairs, waves):
     assert shape(PREC_FP32, DPREFINE, pairs, maxaln, batched=1)[0] == (4 if small else waves)
 
 
+@pytest.mark.parametrize("prec,maxaln,live,waves", [
+    (PREC_FP32, 100, 0, 8), (PREC_FP32, 100, 512, 8), (PREC_FP32, 100, 513, 4), (PREC_FP32, 500, 2560, 8),
+    (PREC_FP32, 500, 2561, 4), (PREC_MIXED, 100, 256, 8), (PREC_MIXED, 100, 257, 4), (PREC_MIXED, 211, 900, 4),
+    (PREC_MIXED, 650, 1280, 8), (PREC_MIXED, 650, 1281, 4)])
+def test_final_waves_follow_the_pairs_left(prec, maxaln, live, waves):
+    """Not one size for every chunk: 900 frames of an ensemble fill the CUs
+    with workgroups of half the size."""
+    for mode in (1, 2, 3, 4):
+        assert shape(prec, mode, live, maxaln)[0] == waves
+    for mode in (5, 6):                         # FULLA: 768 slots a pair
+        assert shape(prec, mode, live, maxaln)[0] == 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [PREC_FP32, PREC_MIXED], ids=["fp32", "mixed"])
+def test_final_stage_with_both_workgroups(prec):
+    """700 copies of a chain (4-wave workgroups in the plain form, 8-wave ones
+    in the batched form) against the same copies in two chunks of 350 and, in
+    four, of 175."""
+    rng = np.random.default_rng(9)
+    x = synth.chain(41, 97)
+    rs = [synth.rigid_copy(rng, x, 0.2 + 0.3 * (i % 8)) for i in range(700)]
+    q, r = Chunk.from_structures([x], ["A" * 97]), Chunk.from_structures(rs, ["A" * 97] * 700)
+    want = batched_equals_plain(q, r, precision=prec)
+    live = int((want.alndata[..., 4] > 0).sum())
+    assert shape(prec, 2, live, 97)[0] == 4 and shape(prec, 2, 175, 97)[0] == 8
+    for n in (350, 175):
+        for k in range(0, 700, n):
+            part = r.subset(range(k, k + n))
+            with GtaBatch(0, default_options(precision=prec), max_qrys=1, max_qry_poss=97, max_refs=n,
+                          max_ref_poss=part.nposs) as b:
+                b.TransferQueryPMDataToDevice(q)
+                b.TransferCPMDataToDevice(part)
+                g = b.ProcessBlock()
+            assert np.array_equal(g.alndata, want.alndata[:, k:k + n])
+            assert np.array_equal(g.tfms, want.tfms[:, k:k + n])
+
+
 @pytest.mark.parametrize("mode", range(8))
 @pytest.mark.parametrize("pairs", [1, 1000, 100000, 1000000])
 def test_split_workgroups_leave_room_for_16_waves(mode, pairs):
