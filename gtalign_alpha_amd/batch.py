@@ -82,6 +82,8 @@ def lib():
         L.gta_test_set_dp_grid.restype = C.c_int
         L.gta_test_set_split.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int]
         L.gta_test_set_split.restype = C.c_int
+        L.gta_test_solve_op.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
+        L.gta_test_solve_op.restype = C.c_int
         L.gta_test_refine_shape.argtypes = [C.c_int] * 3 + [C.c_longlong] + [C.c_int] * 3 + [C.c_void_p]
         L.gta_test_refine_shape.restype = C.c_int
         L.gta_test_pair_score.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
@@ -190,6 +192,15 @@ class GtaBatch:
         b = np.ascontiguousarray(d2, np.float32)
         out = np.empty_like(a)
         self._check(lib().gta_test_pair_score(self._h, a.ctypes.data, b.ctypes.data, a.size, out.ctypes.data))
+        return out
+
+    def solve_op(self, kind, a, b=None):
+        """The solve's square root (kind 0), reciprocal (1) or division (2) for
+        arrays of operands (testing hook, include/gta/gtalign_amd_testing.h)."""
+        a = np.ascontiguousarray(a, np.float32)
+        b = a if b is None else np.ascontiguousarray(b, np.float32)
+        out = np.empty_like(a)
+        self._check(lib().gta_test_solve_op(self._h, kind, a.ctypes.data, b.ctypes.data, a.size, out.ctypes.data))
         return out
 
     def dp_under(self, tfms, gap0=True, gapopen=0.0, usess=False, dpscan=False):

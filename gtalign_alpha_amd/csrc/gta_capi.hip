@@ -1221,23 +1221,35 @@ int gta_test_set_dp_grid(gta_ctx* c, int mode) {
     return GTA_OK;
 }
 
+// the pair score (kind -1) or an operation of the solve (0-2) over host arrays
+static int run_operands(gta_ctx* c, int kind, const float* a, const float* b, int n, float* out) {
+    HIPCHK(c, hipSetDevice(c->device));
+    DevBuf buf;
+    const size_t sz = (size_t)n * sizeof(float);
+    hipError_t e = buf.ensure(3 * sz);
+    if (e != hipSuccess) return fail(c, GTA_ERR_HIP, hipGetErrorString(e));
+    float* d = buf.as<float>();
+    float* o = d + 2 * (size_t)n;
+    int rc = GTA_OK;
+    if ((e = hipMemcpy(d, a, sz, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(d + n, b, sz, hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = kind < 0 ? launch_pair_score(d, d + n, n, o, c->stream)
+                      : launch_solve_op(kind, d, d + n, n, o, c->stream)) != hipSuccess ||
+        (e = hipStreamSynchronize(c->stream)) != hipSuccess ||
+        (e = hipMemcpy(out, o, sz, hipMemcpyDeviceToHost)) != hipSuccess)
+        rc = fail(c, GTA_ERR_HIP, hipGetErrorString(e));
+    buf.release();
+    return rc;
+}
+
 int gta_test_pair_score(gta_ctx* c, const float* d02, const float* d2, int n, float* out) {
     if (!c || !d02 || !d2 || !out || n < 0) return fail(c, GTA_ERR_ARG, "invalid argument");
-    HIPCHK(c, hipSetDevice(c->device));
-    DevBuf b;
-    const size_t sz = (size_t)n * sizeof(float);
-    hipError_t e = b.ensure(3 * sz);
-    if (e != hipSuccess) return fail(c, GTA_ERR_HIP, hipGetErrorString(e));
-    float* a = b.as<float>();
-    int rc = GTA_OK;
-    if ((e = hipMemcpy(a, d02, sz, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(a + n, d2, sz, hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = launch_pair_score(a, a + n, n, a + 2 * (size_t)n, c->stream)) != hipSuccess ||
-        (e = hipStreamSynchronize(c->stream)) != hipSuccess ||
-        (e = hipMemcpy(out, a + 2 * (size_t)n, sz, hipMemcpyDeviceToHost)) != hipSuccess)
-        rc = fail(c, GTA_ERR_HIP, hipGetErrorString(e));
-    b.release();
-    return rc;
+    return run_operands(c, -1, d02, d2, n, out);
+}
+
+int gta_test_solve_op(gta_ctx* c, int kind, const float* a, const float* b, int n, float* out) {
+    if (!c || !a || !b || !out || n < 0 || kind < 0 || kind > 2) return fail(c, GTA_ERR_ARG, "invalid argument");
+    return run_operands(c, kind, a, b, n, out);
 }
 
 int gta_test_valu_calibration(gta_ctx* c, int blocks, int iters, int kind, int lanes, double* seconds) {

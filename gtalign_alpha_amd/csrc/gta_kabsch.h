@@ -21,11 +21,14 @@ template <> __device__ __forceinline__ double t_sqrt<double>(double x) { return 
 __device__ __forceinline__ float t_abs(float x) { return fabsf(x); }
 __device__ __forceinline__ double t_abs(double x) { return fabs(x); }
 // The solve's divisions and square roots, correctly rounded as the plain
-// operators are, without their scaling and special cases (operands here are
-// normal and far from the exponent limits).  Checked on gfx950 against the
-// operators: the square root over every mantissa at both exponent parities, the
-// reciprocal over every mantissa, the division over every pair of mantissas
-// (div_rn_pos, gta_device.h).  In single precision a square root takes 5
+// operators are, without their scaling and special cases.  Radicands and
+// divisors are positive, normal and far from the exponent limits.  Equal to the
+// operators' bits on gfx950: the square root over every mantissa at both exponent
+// parities, the reciprocal over every mantissa, the division over every pair of
+// mantissas (div_rn_pos, gta_device.h).  A numerator may be zero or tiny beside
+// the others: a quotient of -0 becomes +0, and below 2^-100 the residual is
+// itself rounded and the quotient may be off by an ulp or two, at 10^-12 of the
+// matrix's mean magnitude or less.  In single precision a square root takes 5
 // instructions instead of 15, its reciprocal 8 instead of 26, a further
 // division by the same number 3 instead of 11.
 __device__ __forceinline__ float t_sqrt_pos(float x) {

@@ -2399,6 +2399,15 @@ hipError_t launch_pair_score(const float* d02, const float* d2, int n, float* ou
     if (n > 0) hipLaunchKernelGGL(k_pair_score, dim3(blocks_for(n, 256)), dim3(256), 0, st, d02, d2, n, out);
     return hipGetLastError();
 }
+// the solve's short division (kind 2), square root (0) and reciprocal (1)
+__global__ void k_solve_op(int kind, const float* a, const float* b, int n, float* out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = kind == 0 ? t_sqrt_pos(a[i]) : kind == 1 ? t_rcp(a[i]) : t_div(a[i], b[i], t_rcp(b[i]));
+}
+hipError_t launch_solve_op(int kind, const float* a, const float* b, int n, float* out, hipStream_t st) {
+    if (n > 0) hipLaunchKernelGGL(k_solve_op, dim3(blocks_for(n, 256)), dim3(256), 0, st, kind, a, b, n, out);
+    return hipGetLastError();
+}
 // VALU issue-rate calibration for the instruction counters: the first `lanes`
 // lanes of every wave run `iters` iterations of 8 independent chains of one
 // instruction kind K, so each wave issues exactly 8 VALU instructions of that

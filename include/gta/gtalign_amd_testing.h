@@ -87,6 +87,12 @@ int gta_test_refine_shape(int prec, int mode, int ncu, long long pairs, int maxa
  * division does). */
 int gta_test_pair_score(gta_ctx* ctx, const float* d02, const float* d2, int n, float* out);
 
+/* The superposition solve's single-precision square root (kind 0, of a),
+ * reciprocal (1, of a) and division (2, a / b) for n caller-given operands: out[i]
+ * receives the device's value (correctly rounded over the ranges that the solve
+ * uses). */
+int gta_test_solve_op(gta_ctx* ctx, int kind, const float* a, const float* b, int n, float* out);
+
 /* VALU issue-rate calibration for the instruction counters: `blocks`
  * workgroups of 256 lanes; the first `lanes` (1-64) lanes of every wave run
  * `iters` iterations of 8 independent chains of one instruction kind:
