@@ -230,10 +230,19 @@ int gta_dp_cell_counts(const gta_ctx* ctx, double* useful, double* launched);
 /* ---- DP launch-form autotuning (no counterpart in the reference, whose DP
  * tile shape and launch geometry are fixed, dpw_btck.cu:78-615) ------------
  * Each pair's DP fill runs as one wave, as one workgroup of 4, 8 or 16 waves,
- * or pipelined over the whole device.  Off (the default), large pairs take
- * the grid form when they number at most half the compute units and the
- * W-wave form otherwise, and small chunks the W-wave form.  On, pairs of >= 4
- * strips of 64 rows and >= 2^18 cells are grouped by length bucket (log2 of the strip count, log2 of the
+ * or pipelined over the whole device.  Off (the default):
+ *  - large pairs (>= 4,194,304 cells, >= 16 groups of 64 query rows, reference of
+ *    >= 256) take the whole device when they number at most half the compute
+ *    units, a workgroup when they number at most 16 per compute unit, and one
+ *    wave otherwise;
+ *  - in a chunk of at most two pairs per compute unit, the other pairs that a
+ *    workgroup is estimated to fill in 3/4 of one wave's time or less take one;
+ *  - in a larger chunk whose longest fill is estimated to outlast the device's
+ *    share of all fills (a third of it with a prescreen), the longest pairs that
+ *    make up a tenth of the share take the whole device;
+ *  - every other pair takes one wave.
+ * On, pairs of >= 4 groups of 64 rows and >= 2^18 cells are grouped by length
+ * bucket (log2 of the number of groups, log2 of the
  * reference length, log2 of the bucket's pair count); at the first
  * gta_process on a chunk pair, each bucket without a cached choice is timed
  * over the candidate forms (whole-chunk fills, identity superpositions) and

@@ -39,20 +39,20 @@ int gta_test_dp(gta_ctx* ctx, const float* tfms, int gap0, float gapopen, int us
 int gta_test_dp_score(gta_ctx* ctx, const float* tfms, const int* slotflags, int nslots, int gap0,
                       float gapopen, float* scores);
 
-/* Thresholds of the DP's size buckets: a pair is filled by a workgroup of
- * several waves (strips pipelined down the query) when Lq*Lr >= min_cells,
- * it has at least min_strips groups of 64 rows and Lr >= 256; otherwise by
- * one wave.  Before the first call: 4,194,304 cells and 16 groups, and in
- * chunks of at most two pairs per CU every pair that several waves fill in 3/4
- * of the time or less.  Takes effect at the next gta_process / gta_test_dp.
- * Lets tests drive the multi-wave fill on moderate sizes. */
+/* Thresholds of the DP's size buckets: a pair is large when Lq*Lr >= min_cells,
+ * it has at least min_strips groups of 64 rows and Lr >= 256.  After this call
+ * large pairs are filled by a workgroup of several waves (strips pipelined down
+ * the query), however many they are, or by the whole device
+ * (gta_test_set_dp_grid), and all others by one wave; before it, the rules that
+ * gta_set_autotune states hold.  Takes effect at the next gta_process /
+ * gta_test_dp.  Lets tests drive the multi-wave fill on moderate sizes. */
 int gta_test_set_dp_buckets(gta_ctx* ctx, long long min_cells, int min_strips);
 
-/* Pairs of the multi-wave bucket above are filled by the whole device
- * instead (one-wave workgroups pipelining the pair's strips through global
- * memory) when mode is 1, never when 2, and when they number at most half
- * the device's compute units when 0 (the default).  Takes effect at the next
- * gta_process / gta_test_dp. */
+/* Large pairs (above) are filled by the whole device (one-wave workgroups
+ * pipelining the pair's strips through global memory) when mode is 1, never
+ * when 2, and when they number at most half the device's compute units when 0
+ * (the default).  2 also keeps the longest pairs of larger chunks off it.  Takes
+ * effect at the next gta_process / gta_test_dp. */
 int gta_test_set_dp_grid(gta_ctx* ctx, int mode);
 
 /* DP launch forms of the resident chunk pair as of the last gta_process or
