@@ -52,7 +52,7 @@ KERNEL_NAMES = {
     "refine_gapless": "gta::k_refine_gapless<0>",
     "dp": "gta::k_dp<0, true/false> (29 of 30 launches; 1 is k_dp<1, false>)",
     "refine_dp": "gta::k_refine_dp<0, 0, 1> (RM_DPREFINE, 1-wave workgroups on the bench's chunks)",
-    "refine_final": "gta::k_refine_dp<0, 1..4, 8> (final and production phases)",
+    "refine_final": "gta::k_refine_dp<0, 1..4, 4> (final and production phases)",
 }
 
 

@@ -34,11 +34,11 @@ enum { BT_STOP = 0, BT_LEFT = 1, BT_UP = 2, BT_DIAG = 3 };  // gproc.h:180-185
 // covariance record: 9 cross terms, query sum, reference sum, count
 enum { CCM00 = 0, CVq0 = 9, CVr0 = 12, NALN = 15, NCC = 16 };
 
-// waves per workgroup of the gapless refinement and the log search (one pair,
-// or one part of a pair, per workgroup; DPRefine's depend on the chunk's size,
-// the final stage's follow): two waves keep the share of a workgroup's time spent
-// waiting for its last slots small and leave LDS to stage alignments of up to
-// 682 positions
+// waves per workgroup of the gapless refinement, the log search and split
+// pairs (one pair, or one part of a pair, per workgroup; DPRefine's and the
+// final stage's: refine_shape, gta_launch.h): two waves keep the share of a
+// workgroup's time spent waiting for its last slots small and leave LDS to
+// stage alignments of up to 682 positions
 constexpr int REFINE_WAVES = 2;
 // and the most of the final stage's refinements (final_waves, gta_launch.h)
 constexpr int FINAL_WAVES = 8;
