@@ -16,11 +16,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1301,7 +1301,7 @@ struct SectionClear {
     void start(char* p, size_t n) {
         try {
             t = std::thread([p, n] { memset(p, 0, n); });
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {       // no thread or no memory for one
             memset(p, 0, n);
         }
     }
